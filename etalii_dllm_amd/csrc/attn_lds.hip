@@ -136,7 +136,8 @@ __device__ __forceinline__ void wait_stage() {
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPending) : "memory");
 }
 
-__device__ __forceinline__ void workgroup_barrier() { asm volatile("s_barrier" ::: "memory"); }
+// Ends a stage: this wave's LDS reads of it have returned before anyone's next copies may overwrite it.
+__device__ __forceinline__ void workgroup_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Where the next stage's copies start, as wave-uniform values (scalar registers): step l, A's row of step l (from
 // column i0), and B's row of query l / group (head 0 of the group; B rows are (query, head of the group) pairs) with

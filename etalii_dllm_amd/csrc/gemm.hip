@@ -208,7 +208,8 @@ __device__ __forceinline__ void wait_stage() {
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kPending) : "memory");
 }
 
-__device__ __forceinline__ void workgroup_barrier() { asm volatile("s_barrier" ::: "memory"); }
+// Ends a stage: this wave's LDS reads of it have returned before anyone's next copies may overwrite it.
+__device__ __forceinline__ void workgroup_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 
 // Issues the copies of stage rows l .. l + kChunk - 1 (rows past `last` repeat row `last`; they are never read).
@@ -704,10 +705,10 @@ __device__ __forceinline__ void maccumulate(const GemmParams& p, MStage<kA, kBI,
             wait_stage<0>();
         }
         mstage_full<kA, kBI, kBJ>(st[c & 1], wi, wj, lane, acc);
-        // every wave has issued its reads of the stage before the next issue overwrites it. The compiler places the
-        // stage's last MFMAs, and the waits for their fragment reads, after this barrier; those reads are already in
-        // the CU's LDS pipeline, and the copy that refills the buffer is issued after the barrier and writes only
-        // when its data returns from memory. (Waiting for the reads here cost 0.45% of the c3 step.)
+        // Every wave's reads of the stage have returned before the next issue overwrites it. The wait is needed: the
+        // compiler places the stage's last MFMAs, and the waits for their fragments, after this barrier, and reads only
+        // issued could be overtaken by a copy that another wave issues after it (a step of 450 such launches gave other
+        // weights about once in a hundred; the wait costs 0.5% of these launches).
         workgroup_barrier();
     }
     if (tail) {
