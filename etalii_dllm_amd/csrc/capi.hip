@@ -18,10 +18,21 @@ namespace {
 
 hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
+// The int8 matmul path's scratch for one plain matmul I x J over L.
+size_t split_ws(size_t I, size_t J, size_t L, int a_kind) {
+    GemmCall g;
+    g.a_kind = a_kind;
+    g.I = static_cast<int64_t>(I);
+    g.J = static_cast<int64_t>(J);
+    g.l1 = static_cast<int64_t>(L);
+    return split_gemm_bytes(g);
+}
+
 size_t linear_ws(size_t rows, size_t in, size_t out) {
     Layout l;
     l.add<double>(in * static_cast<size_t>(padded_rows(rows)));  // x^T as double
     l.add<float>(in * out);                                         // W^T
+    l.add<char>(split_ws(rows, out, in, 2));
     return l.bytes;
 }
 
@@ -29,6 +40,7 @@ size_t linear_backward_ws(size_t rows, size_t in, size_t out) {
     Layout l;
     l.add<double>(rows * static_cast<size_t>(padded_rows(out)));  // dy as double [rows][out_pad]
     l.add<double>(out * static_cast<size_t>(padded_rows(rows)));  // dy^T as double [out][rows_pad]
+    l.add<char>(std::max(split_ws(rows, in, out, 2), split_ws(out, in, rows, 1)));  // one of the two matmuls at a time
     return l.bytes;
 }
 
@@ -128,15 +140,24 @@ int dllm_hip_linear(const float* x, const float* w, const float* bias, float* ou
     const int64_t R = static_cast<int64_t>(rows), K = static_cast<int64_t>(in), N = static_cast<int64_t>(out_f);
     double* xT = c.take<double>(K * padded_rows(R));
     float* wT = c.take<float>(K * N);
+    const size_t split_cap = split_ws(rows, out_f, in, 2);
+    char* split = c.take<char>(split_cap);
     DLLM_REQUIRE(!c.overflow, "workspace layout overflow");
     const hipStream_t s = as_stream(stream);
-    DLLM_TRY(launch_transpose_f32(w, N, K, wT, s));
     GemmCall g;
     if (K % 4 == 0 && N % 4 == 0 && aligned16(x)) {  // the matmul reads x itself
         g.Af = x;
         g.a_kind = 2;
         g.lda = K;
+        if (aligned16(w)) {  // and, on the int8 path, w itself: wT is filled only for what that path hands back
+            g.Bt = w;
+            g.ldbt = K;
+            g.bt_transpose = wT;
+        } else {
+            DLLM_TRY(launch_transpose_f32(w, N, K, wT, s));
+        }
     } else {
+        DLLM_TRY(launch_transpose_f32(w, N, K, wT, s));
         DLLM_TRY(launch_to_double(x, R, K, K, nullptr, 0, xT, padded_rows(R), s));
         g.A = xT;
         g.lda = padded_rows(R);
@@ -150,6 +171,8 @@ int dllm_hip_linear(const float* x, const float* w, const float* bias, float* ou
     g.l0 = 0;
     g.l1 = K;
     g.bias = bias;
+    g.split_scratch = split;
+    g.split_cap = split_cap;
     return launch_gemm(g, s);
 }
 
@@ -293,6 +316,8 @@ int dllm_hip_linear_backward(const float* x, const float* w, const float* dy, fl
     const int64_t R = static_cast<int64_t>(rows), K = static_cast<int64_t>(in), N = static_cast<int64_t>(out_f);
     double* dy_d = c.take<double>(R * padded_rows(N));
     double* dyT_d = c.take<double>(N * padded_rows(R));
+    const size_t split_cap = std::max(split_ws(rows, in, out_f, 2), split_ws(out_f, in, rows, 1));
+    char* split = c.take<char>(split_cap);
     DLLM_REQUIRE(!c.overflow, "workspace layout overflow");
     const hipStream_t s = as_stream(stream);
     // the matmuls read dy itself when its rows are whole 16-byte chunks; otherwise as doubles
@@ -322,6 +347,8 @@ int dllm_hip_linear_backward(const float* x, const float* w, const float* dy, fl
             g.J = K;
             g.l0 = 0;
             g.l1 = N;
+            g.split_scratch = split;
+            g.split_cap = split_cap;
             DLLM_TRY(launch_gemm(g, s));
         }
     }
@@ -346,6 +373,8 @@ int dllm_hip_linear_backward(const float* x, const float* w, const float* dy, fl
             g.J = K;
             g.l0 = 0;
             g.l1 = R;
+            g.split_scratch = split;
+            g.split_cap = split_cap;
             DLLM_TRY(launch_gemm(g, s));
         }
     }

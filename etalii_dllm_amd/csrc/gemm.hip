@@ -33,8 +33,9 @@
 #include <vector>
 
 #include "common.h"
-#include "lds_copy.h"
+#include "gemm_split.h"
 #include "kernels.h"
+#include "lds_copy.h"
 
 namespace dllm_hip {
 
@@ -72,6 +73,8 @@ struct GemmParams {
     const float* Af;  // float A operands: [L][lda] (A rows) or [I][lda] (A transposed: Af[i][l] = A[l][i])
     const float* seg_weight;  // segmented mode: per-window factors on each window's result (null: none)
     const float* seg_rowscale;  // segmented mode: per-row factors on each window's result, before seg_weight
+    int64_t ld_addrow;  // row stride of seg_addrow
+    const uint8_t* only = nullptr;  // matrix-core kernel: the tiles to compute, [window][row tile][column tile] (null: all)
 };
 
 // The raw B values of row l for this lane's 4 columns. Lanes past J read a clamped in-bounds column instead (their
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         for (int q = 0; q < kTileI; ++q) {
             const int64_t i = i0 + q;
             if (i >= p.I) break;
-            const int arow = p.seg_addrow ? p.seg_addrow[static_cast<int64_t>(s) * p.I + i] : -1;
+            const int arow = p.seg_addrow ? p.seg_addrow[static_cast<int64_t>(s) * p.ld_addrow + i] : -1;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const int64_t j = j0 + c;
@@ -432,7 +435,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         for (int q = 0; q < kTileI; ++q) {
             const int64_t i = i0 + q;
             if (i >= p.I) break;
-            const int arow = p.seg_addrow ? p.seg_addrow[static_cast<int64_t>(s) * p.I + i] : -1;
+            const int arow = p.seg_addrow ? p.seg_addrow[static_cast<int64_t>(s) * p.ld_addrow + i] : -1;
             const auto out = global_ptr(out_base) + i * ld_out + j0;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -759,6 +762,7 @@ gemm_mfma_kernel(GemmParams p, int64_t gx, int64_t gy, int64_t gz, const GemmPar
     const int64_t rows_in_group = gy - first < kGroupRows ? gy - first : kGroupRows;
     const int64_t by = first + (t % (kGroupRows * gx)) % rows_in_group;
     const int64_t bx = (t % (kGroupRows * gx)) / rows_in_group;
+    if (!kGrouped && p.only && !p.only[(bz * gy + by) * gx + bx]) return;
     const int64_t i_blk = by * T::I, j_blk = bx * T::J;
     const int64_t iw = i_blk + wi * 16 * kBI;  // this wave's first row
     const int64_t jw = j_blk + wj * 16 * kBJ + (lane & 15);
@@ -856,7 +860,7 @@ gemm_mfma_kernel(GemmParams p, int64_t gx, int64_t gy, int64_t gz, const GemmPar
             if (p.seg_addrow) {
                 int arow[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) arow[r] = seg_addrow[static_cast<int64_t>(s) * p.I + ic[r]];
+                for (int r = 0; r < 4; ++r) arow[r] = seg_addrow[static_cast<int64_t>(s) * p.ld_addrow + ic[r]];
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -956,8 +960,10 @@ __global__ __launch_bounds__(256) void to_double_kernel(const float* __restrict_
 
 // dst[c][r] = src[r][c] in float (the forward pass's W^T).
 __global__ __launch_bounds__(256) void transpose_f32_kernel(const float* __restrict__ src, int64_t rows, int64_t cols,
-                                                            float* __restrict__ dst) {
+                                                            float* __restrict__ dst,
+                                                            const uint32_t* __restrict__ needed) {
     __shared__ float tile[64][65];
+    if (needed && *needed == 0) return;
     const int64_t r0 = static_cast<int64_t>(blockIdx.y) * 64;
     const int64_t c0 = static_cast<int64_t>(blockIdx.x) * 64;
     const int tx = threadIdx.x & 63;
@@ -1050,10 +1056,12 @@ bool mfma_shape(const GemmCall& g) {
 GemmParams params_of(const GemmCall& g) {
     return GemmParams{g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.I, g.J, g.l0, g.l1, g.seg, g.nseg, g.bias, g.addsrc,
                       g.ld_add, g.seg_addend, g.seg_addrow, g.ld_seg_add, nullptr, g.Af, g.seg_weight,
-                      g.seg_rowscale};
+                      g.seg_rowscale, g.ld_addrow ? g.ld_addrow : g.I, nullptr};
 }
 
 }  // namespace
+
+int64_t gemm_split_rows(const GemmCall& g) { return mfma_shape(g) ? split_plan(g).rows : 0; }
 
 bool gemm_mfma_shape(const GemmCall& g) { return g.a_kind != kADouble && mfma_shape(g); }
 
@@ -1328,6 +1336,23 @@ int launch_gemm(const GemmCall& g, hipStream_t stream) {
             DLLM_REQUIRE(g.seg == nullptr && g.l0 == 0 && g.l1 % 4 == 0 && g.l1 >= 4 && g.lda >= g.l1,
                          "transposed float A needs a plain reduction over whole 16-byte chunks");
     }
+    const SplitPlan split = split_plan(g);
+    if (split.rows > 0 && split.rows < g.I) {  // row blocks that share B's split
+        for (int64_t i0 = 0; i0 < g.I; i0 += split.rows) {
+            GemmCall b = g;
+            b.I = std::min(split.rows, g.I - i0);
+            b.Af = ak == kAFloatT ? g.Af + i0 * g.lda : g.Af + i0;
+            b.C = g.C + i0 * g.ldc;
+            if (g.addsrc) b.addsrc = g.addsrc + i0 * g.ld_add;
+            if (g.seg_addrow) b.seg_addrow = g.seg_addrow + i0;
+            b.ld_addrow = g.ld_addrow ? g.ld_addrow : g.I;
+            if (g.seg_rowscale) b.seg_rowscale = g.seg_rowscale + i0;
+            b.split_share = 2;
+            b.split_ready = i0 > 0 && gemm_split_rows(b) == b.I;
+            DLLM_TRY(launch_gemm(b, stream));
+        }
+        return kOk;
+    }
     if (vec && (ak != kADouble || ((g.lda % 2 == 0) && (reinterpret_cast<uintptr_t>(g.A) % 16 == 0)))) {
         const bool mfma = ak != kADouble;
         int64_t gx = mfma ? ceil_div(g.J, MTile<4, 4>::J) : ceil_div(g.J, kTileJ);
@@ -1342,7 +1367,22 @@ int launch_gemm(const GemmCall& g, hipStream_t stream) {
         // matrix-core tiles: 128 x 128, or 64 x 64 / 32 x 32 when the larger tiles' grid leaves CUs idle (128 x 192
         // tiles, which fit a [rows x 1536] output in one round of the 512 workgroup slots, measured slower)
         int tile = 4;
-        if (mfma) {
+        if (split.rows > 0) {
+            // the int8 matrix cores decide almost every output; the tiles they hand back run here, one launch whose
+            // other workgroups end at once
+            p.partial = split.parallel ? g.seg_partial : nullptr;
+            gz = split.parallel ? g.nseg : 1;
+            SplitRedo redo;
+            DLLM_TRY(launch_split_gemm(g, p.partial, stream, &redo));
+            if (g.bt_transpose) DLLM_TRY(launch_transpose_f32(g.Bt, g.J, g.l1, g.bt_transpose, stream, redo.tiles));
+            p.only = redo.tile_flags;
+            gx = ceil_div(g.J, redo.tile);
+            gy = ceil_div(g.I, redo.tile);
+            tile = redo.tile / 32;
+        } else if (g.bt_transpose) {
+            DLLM_TRY(launch_transpose_f32(g.Bt, g.J, g.l1, g.bt_transpose, stream));
+        }
+        if (mfma && !p.only) {
             while (tile > 1 && gx * gy * gz < kSmallTilesBelow) {
                 tile /= 2;
                 gx = ceil_div(g.J, 32 * tile);
@@ -1430,11 +1470,12 @@ int launch_transpose_batch(const TransposeJob* device_jobs, const int64_t* devic
     return check_launch("transpose batch");
 }
 
-int launch_transpose_f32(const float* src, int64_t rows, int64_t cols, float* dst, hipStream_t stream) {
+int launch_transpose_f32(const float* src, int64_t rows, int64_t cols, float* dst, hipStream_t stream,
+                         const uint32_t* needed) {
     if (rows == 0 || cols == 0) return kOk;
     dim3 grid(static_cast<unsigned>(ceil_div(cols, 64)), static_cast<unsigned>(ceil_div(rows, 64)));
     DLLM_REQUIRE(grid.y <= 65535u, "too many rows for one transpose launch");
-    hipLaunchKernelGGL(transpose_f32_kernel, grid, dim3(256), 0, stream, src, rows, cols, dst);
+    hipLaunchKernelGGL(transpose_f32_kernel, grid, dim3(256), 0, stream, src, rows, cols, dst, needed);
     return check_launch("transpose");
 }
 

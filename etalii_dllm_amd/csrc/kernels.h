@@ -44,7 +44,27 @@ struct GemmCall {
     // (a_scratch_cap doubles, at least l1 x padded_rows(I)) and the call runs on the VALU kernels with the same bits
     double* a_scratch = nullptr;
     int64_t a_scratch_cap = 0;
+    int64_t ld_addrow = 0;  // row stride of seg_addrow (0: I)
+    // Optional scratch of split_cap bytes (split_gemm_bytes; with less, the call runs in row blocks) for the int8
+    // matrix-core path of large float-A calls (gemm_split.hip, the same bits). seg_max: the longest window (segmented
+    // calls; l1 then holds all windows' rows).
+    void* split_scratch = nullptr;
+    size_t split_cap = 0;
+    int64_t seg_max = 0;
+    // Bt: B's values with l contiguous (Bt[j][l], rows of whole 16-byte chunks), read instead of B by that path.
+    // bt_transpose: B is scratch, to be filled from Bt where the call reads it.
+    const float* Bt = nullptr;
+    int64_t ldbt = 0;
+    float* bt_transpose = nullptr;
+    // Calls in a row on one stream and scratch that share an operand (1: A, 2: B) split it once: split_ready says that
+    // the call before, of the same share, reduction and windows, left it in the scratch.
+    int split_share = 0;
+    bool split_ready = false;
 };
+// The rows of a block of the call on the int8 path: I when it runs there whole, 0 when it does not run there.
+int64_t gemm_split_rows(const GemmCall& g);
+// Scratch bytes of the int8 path for the whole call (0: the shape does not take it).
+size_t split_gemm_bytes(const GemmCall& g);
 // Whether a float-A call runs on the matrix-core kernel (every operand row a whole number of 16-byte chunks).
 bool gemm_mfma_shape(const GemmCall& g);
 
@@ -80,7 +100,9 @@ int launch_gemm_row_group_fill(const void* device_templ, void* device_table, con
 // dst[r][c] = src[r][c] and dstT[c][r] = src[r][c] as doubles (either may be null).
 int launch_to_double(const float* src, int64_t rows, int64_t cols, int64_t lds, double* dst, int64_t ldd,
                      double* dstT, int64_t lddT, hipStream_t stream);
-int launch_transpose_f32(const float* src, int64_t rows, int64_t cols, float* dst, hipStream_t stream);
+// needed: optional device count; the kernel leaves dst alone while it is 0.
+int launch_transpose_f32(const float* src, int64_t rows, int64_t cols, float* dst, hipStream_t stream,
+                         const uint32_t* needed = nullptr);
 // dst = src^T for many matrices in one launch: transpose_batch_tiles fills the n + 1 tile starts (host) and returns
 // the tile count; the jobs and the starts are then passed in device memory.
 struct TransposeJob {

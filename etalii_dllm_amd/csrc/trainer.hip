@@ -208,6 +208,8 @@ struct dllm_hip_trainer {
           *dgate = nullptr, *dup = nullptr, *col_part = nullptr, *col_part_side = nullptr, *emb_rows = nullptr,
           *gemm_part = nullptr;
     int64_t gemm_part_cap = 0;  // floats: per-window partials of the layer weight gradients
+    char* split_mem[2] = {nullptr, nullptr};  // the int8 matmuls' scratch: the step's stream, the side stream
+    size_t split_cap[2] = {0, 0};
     // routed experts: E experts, K per token, EI expert intermediate size; shared buffers of the grouped rows
     int64_t E = 0, K = 0, EI = 0, RK = 0;
     float *xg = nullptr, *dyg = nullptr, *dxg = nullptr, *dweights = nullptr, *dlogits_r = nullptr, *dprob = nullptr,
@@ -626,6 +628,10 @@ struct dllm_hip_trainer {
             gemm_part_cap = W_max * H * std::max<int64_t>({QD, KVD, I, EI, E});
             DLLM_TRY(make(&gemm_part, gemm_part_cap));
         }
+        for (int k = 0; k < 2; ++k) {
+            split_cap[k] = std::min(split_bytes(k == 1), kSplitMax);
+            if (split_cap[k] > 0) DLLM_TRY(make(&split_mem[k], split_cap[k]));
+        }
         DLLM_TRY(make(&emb_rows, R * H));
         DLLM_TRY(make(&inv_rms, R * std::max<int64_t>(heads, 1)));
         DLLM_TRY(make(&inv_mlp, R));
@@ -893,11 +899,63 @@ struct dllm_hip_trainer {
         return kOk;
     }
 
+    // The most scratch an int8 matmul of a full step takes (side: of the layers' weight gradients), and the cap on it:
+    // a larger call runs in row blocks, at 8192 x 151936 logits two for the head's input gradient (768 tiles each) and
+    // three for its weight gradient.
+    static constexpr size_t kSplitMax = size_t{5} << 30;
+
+    size_t split_bytes(bool side_stream) const {
+        size_t most = 0;
+        const int head = c.tie_embeddings ? emb : lm_head;
+        for (size_t i = 0; i < tensors.size(); ++i) {
+            const TensorInfo& t = tensors[i];
+            if (t.wt_offset < 0 || (side_stream && static_cast<int>(i) == head)) continue;
+            GemmCall fwd, dx, dw;
+            fwd.a_kind = dx.a_kind = 2;
+            fwd.I = dx.I = dw.l1 = R_max;
+            fwd.J = dx.l1 = dw.I = t.rows;
+            dx.J = fwd.l1 = dw.J = t.cols;
+            fwd.Bt = dx.Bt = params.as<float>();  // any: the sizes alone count here
+            dw.a_kind = 1;
+            dw.seg = seg_d ? seg_d : reinterpret_cast<const int64_t*>(params.p);
+            dw.nseg = static_cast<int>(W_max);
+            dw.seg_max = T_max;
+            dw.seg_partial = gemm_part;
+            dw.seg_partial_cap = gemm_part_cap;
+            if (!side_stream) most = std::max({most, split_gemm_bytes(fwd), split_gemm_bytes(dx)});
+            most = std::max(most, split_gemm_bytes(dw));
+        }
+        return most;
+    }
+
+    // The call with the int8 path's scratch of its stream.
+    GemmCall with_split(const GemmCall& g, hipStream_t s) const {
+        GemmCall c = g;
+        const int k = side_on && s == side ? 1 : 0;
+        c.split_scratch = split_mem[k];
+        c.split_cap = split_cap[k];
+        return c;
+    }
+
     int gemm(const GemmCall& g, hipStream_t s) {
-        if (!profiling) return launch_gemm(g, s);
+        if (!profiling) return launch_gemm(with_split(g, s), s);
         DLLM_TRY(profile_begin(s));
-        DLLM_TRY(launch_gemm(g, s));
+        DLLM_TRY(launch_gemm(with_split(g, s), s));
         return profile_end(flops_of(g), s);
+    }
+
+    // Matmuls that share operand `share` (1: A, 2: B), back to back on one stream: it is split once.
+    int gemm_shared(const GemmCall* calls, int n, int share, hipStream_t s) {
+        bool ready = false;
+        for (int k = 0; k < n; ++k) {
+            GemmCall g = calls[k];
+            g.split_share = share;
+            g.split_ready = ready;
+            const int64_t rows = gemm_split_rows(with_split(g, s));
+            DLLM_TRY(gemm(g, s));
+            if (rows > 0) ready = rows == g.I;  // in row blocks it leaves their split there
+        }
+        return kOk;
     }
 
     // One launch of a layer's expert matmuls (a group table made by group_rows).
@@ -1025,9 +1083,10 @@ struct dllm_hip_trainer {
                 const size_t gi = static_cast<size_t>(l * kLayerGroups + k);
                 if (ok) DLLM_TRY(gemm_group_prepare(calls, nc, kGroupCap, host.data() + gb * gi, &g));
                 for (int i = 0; i < nc; ++i) grp_flops[gi] += flops_of(calls[i]);
-                // the input-gradient groups only where the separate launches would take small tiles
+                // the input-gradient groups only where the separate launches would take small tiles; none whose first
+                // matmul runs on the int8 path (the others then share its split of the rows)
                 const bool dx_kind = k == kGrpMlpDx || k == kGrpQkvDx;
-                if (!ok || (dx_kind && g.tile == 4)) grp_on[k] = false;
+                if (!ok || (dx_kind && g.tile == 4) || gemm_split_rows(with_split(calls[0], s)) > 0) grp_on[k] = false;
             }
         }
         DLLM_TRY(check_hip(hipStreamSynchronize(s), "group tables"));  // no launch still reads the old tables
@@ -1045,9 +1104,10 @@ struct dllm_hip_trainer {
         const LayerIds& L = layer_ids[static_cast<size_t>(l)];
         Saved& sv = saved[static_cast<size_t>(l)];
         if (grp_on[kGrpQkvFwd] && grp_rows == R) return group_launch(l, kGrpQkvFwd, s);
-        DLLM_TRY(linear_fwd(sv.h1, R, H, L.q, Popt(L.qb), sv.q_raw, nullptr, s));
-        DLLM_TRY(linear_fwd(sv.h1, R, H, L.k, Popt(L.kb), sv.k_raw, nullptr, s));
-        return linear_fwd(sv.h1, R, H, L.v, Popt(L.vb), sv.v, nullptr, s);
+        const GemmCall calls[3] = {fwd_call(sv.h1, R, H, L.q, Popt(L.qb), sv.q_raw, nullptr),
+                                   fwd_call(sv.h1, R, H, L.k, Popt(L.kb), sv.k_raw, nullptr),
+                                   fwd_call(sv.h1, R, H, L.v, Popt(L.vb), sv.v, nullptr)};
+        return gemm_shared(calls, 3, 1, s);
     }
 
     // out[R][N] (+)= x[R][K] @ W^T (+ bias); the matmul reads x itself (A transposed: A[k][r] = x[r][k]).
@@ -1065,6 +1125,8 @@ struct dllm_hip_trainer {
         g.lda = K;
         g.B = WT(w_id);
         g.ldb = N;
+        g.Bt = P(w_id);
+        g.ldbt = K;
         g.C = out;
         g.ldc = N;
         g.I = R;
@@ -1092,6 +1154,8 @@ struct dllm_hip_trainer {
         g.lda = t.rows;
         g.B = P(w_id);
         g.ldb = t.cols;
+        g.Bt = WT(w_id);
+        g.ldbt = t.rows;
         g.C = out;
         g.ldc = t.cols;
         g.I = R;
@@ -1132,6 +1196,9 @@ struct dllm_hip_trainer {
         g.nseg = nseg;
         g.l0 = 0;
         g.l1 = seg ? rows : seg_host.back();
+        if (!seg)
+            for (size_t w = 0; w + 1 < seg_host.size(); ++w)
+                g.seg_max = std::max(g.seg_max, seg_host[w + 1] - seg_host[w]);
         g.seg_addrow = addrow_;
         g.seg_addend = addend;
         g.ld_seg_add = K;
@@ -1331,8 +1398,9 @@ struct dllm_hip_trainer {
         if (grp_on[kGrpMlpFwd] && grp_rows == R) {
             DLLM_TRY(group_launch(l, kGrpMlpFwd, s));
         } else {
-            DLLM_TRY(linear_fwd(sv.h2, R, H, L.gate, nullptr, sv.gate, nullptr, s));
-            DLLM_TRY(linear_fwd(sv.h2, R, H, L.up, nullptr, sv.up, nullptr, s));
+            const GemmCall calls[2] = {fwd_call(sv.h2, R, H, L.gate, nullptr, sv.gate, nullptr),
+                                       fwd_call(sv.h2, R, H, L.up, nullptr, sv.up, nullptr)};
+            DLLM_TRY(gemm_shared(calls, 2, 1, s));
         }
         DLLM_TRY(launch_swiglu_forward(sv.gate, sv.up, sv.gate_act, sv.product, R * I, s, act()));
         if (post_norms()) {  // x_out = x_mid + post_norm(mlp)
@@ -1370,8 +1438,13 @@ struct dllm_hip_trainer {
             DLLM_TRY(side_wait(kSideMlp, s));  // the previous layer's gate and up dW read dgate, dup
             DLLM_TRY(launch_swiglu_backward(sv.gate, sv.up, sv.gate_act, dproduct, dgate, dup, R * I, s, act()));
             DLLM_TRY(side_fork_from(s, &ws));
-            DLLM_TRY(linear_dw(dgate, I, sv.h2, H, nseg, G(L.gate), nullptr, nullptr, ws));
-            DLLM_TRY(linear_dw(dup, I, sv.h2, H, nseg, G(L.up), nullptr, nullptr, ws));
+            {
+                GemmCall calls[2];
+                int n = 0;
+                if (grad_wanted(G(L.gate))) calls[n++] = dw_call(dgate, I, sv.h2, H, nseg, G(L.gate), nullptr, nullptr);
+                if (grad_wanted(G(L.up))) calls[n++] = dw_call(dup, I, sv.h2, H, nseg, G(L.up), nullptr, nullptr);
+                DLLM_TRY(gemm_shared(calls, n, 2, ws));
+            }
             DLLM_TRY(side_mark(kSideMlp));
             DLLM_TRY(side_wait(kSideNormMlp, s));  // the previous layer's mlp norm dW reads dh
             if (grp_on[kGrpMlpDx] && grp_rows == R) {
@@ -1434,9 +1507,17 @@ struct dllm_hip_trainer {
         const int bs_[3] = {L.qb, L.kb, L.vb};
         const int64_t ns[3] = {QD, KVD, KVD};
         DLLM_TRY(side_fork_from(s, &ws));
+        {
+            GemmCall calls[3];
+            int n = 0;
+            for (int p = 0; p < 3; ++p) {
+                if (!grad_wanted(G(ws_[p]))) continue;
+                calls[n] = dw_call(ds[p], ns[p], sv.h1, H, nseg, G(ws_[p]), nullptr, nullptr);
+                calls[n++].seg_rowscale = unfold_scale(ws_[p]);
+            }
+            DLLM_TRY(gemm_shared(calls, n, 2, ws));
+        }
         for (int p = 0; p < 3; ++p) {
-            DLLM_TRY(linear_dw(ds[p], ns[p], sv.h1, H, nseg, G(ws_[p]), nullptr, nullptr, ws, nullptr, -1,
-                               unfold_scale(ws_[p])));
             if (bs_[p] >= 0 && grad_wanted(G(bs_[p])))
                 DLLM_TRY(launch_column_sums(0, ds[p], nullptr, nullptr, ns[p], seg_host.data(), nseg,
                                             ws == s ? col_part : col_part_side, G(bs_[p]), ws, window_weights(),

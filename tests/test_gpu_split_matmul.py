@@ -1,0 +1,82 @@
+"""GPU parity of the matmuls' int8 matrix-core path (csrc/gemm_split.hip): whole outputs against the same calls in pieces
+too small for that path (each output's bits do not depend on the call around it), and sampled rows against the oracle,
+bit for bit. Sizes off the path's 64 x 64 tiles, 64-l steps and 256-l parts; operands with ordinary and very wide rows,
+exact ties, zero rows, infinities and NaNs, so that every way an output is decided is taken."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K():
+    from etalii_dllm_amd import kernels
+
+    return kernels
+
+
+def operand(kind: str, seed: int, rows: int, cols: int) -> np.ndarray:
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((rows, cols)).astype(np.float32)
+    if kind == "tail":  # a few bits per row lost below the sixth digit
+        x = x * np.exp(1.5 * rng.standard_normal((rows, cols))).astype(np.float32)
+    elif kind == "wide":  # rows and columns of very different size, and values from 1e-30 to 1e10 inside some
+        x = x * np.power(10.0, rng.integers(-12, 9, (rows, 1))).astype(np.float32)
+        x[::5] *= np.power(10.0, rng.integers(-18, 2, (len(x[::5]), cols))).astype(np.float32)
+    elif kind == "ties":  # sums that are small integers: exact zeros, ties of the rounding
+        x = rng.integers(-3, 4, (rows, cols)).astype(np.float32)
+        x[:, 0] = 4096.0 * rng.integers(-1024, 1025, rows)
+        x[::3, 1] = 2.0 ** -12
+    elif kind == "special":
+        x[3] = 0.0
+        x[:, 5] = 0.0
+        x[70, 11], x[71, 12], x[200, 13] = np.inf, -np.inf, np.nan
+        x[130] = np.float32(1e-42) * x[130]
+        x[131] = np.float32(3e37) * np.sign(x[131])
+    return np.ascontiguousarray(x)
+
+
+KINDS = ["gauss", "tail", "wide", "ties", "special"]
+
+
+def assert_same(a: np.ndarray, b: np.ndarray, what: str) -> None:
+    nan = np.isnan(a) & np.isnan(b)
+    bad = (a.view(np.uint32) != b.view(np.uint32)) & ~nan
+    assert not bad.any(), (what, int(bad.sum()), a.size, np.argwhere(bad)[:4].tolist())
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("rows,inf,outf", [(2049, 1540, 4868), (1000, 8196, 1348), (4100, 516, 5444)])
+def test_linear(K, kind, rows, inf, outf):
+    x, w = operand(kind, 1, rows, inf), operand("gauss" if kind == "special" else kind, 2, outf, inf)
+    b = operand("gauss", 3, 1, outf)[0]
+    got = K.linear(x, w, b)
+    parts = [K.linear(x[i:i + 256], w[j:j + 512], b[j:j + 512]) for i in range(0, rows, 256)
+             for j in range(0, outf, 512)]
+    nj = -(-outf // 512)
+    want = np.concatenate([np.concatenate(parts[k * nj:(k + 1) * nj], axis=1) for k in range(-(-rows // 256))])
+    assert_same(got, want, "linear")
+    pick = np.array([0, 3, 70, 130, 131, rows - 1])
+    assert_same(got[pick][:, -70:], O.oracle_kernels().linear(x[pick], w[-70:].copy(), b[-70:].copy()), "oracle")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("rows,inf,outf", [(2051, 900, 4868), (8191, 1028, 1540)])
+def test_linear_backward(K, kind, rows, inf, outf):
+    x, w = operand("gauss", 4, rows, inf), operand("gauss", 5, outf, inf)
+    dy = operand(kind, 6, rows, outf)
+    dx, dw, db = K.linear_backward(x, w, dy, with_bias=True)
+    want = np.concatenate([K.linear_backward(x[i:i + 128], w, dy[i:i + 128])[0] for i in range(0, rows, 128)])
+    assert_same(dx, want, "dx")
+    pieces = [K.linear_backward(x, w[j:j + 128], np.ascontiguousarray(dy[:, j:j + 128]), with_bias=True)
+              for j in range(0, outf, 128)]
+    assert_same(dw, np.concatenate([p[1] for p in pieces]), "dw")
+    assert_same(db, np.concatenate([p[2] for p in pieces]), "db")
+    cols = np.array([0, 11, 12, outf - 1])
+    ora = O.oracle_kernels().linear_backward(x, w[cols].copy(), dy[:, cols].copy())
+    assert_same(dw[cols], ora[1], "oracle dw")
