@@ -8,6 +8,7 @@
 #include "common.h"
 #include "devmath.h"
 #include "kernels.h"
+#include "lds_copy.h"
 
 namespace dllm_hip {
 
@@ -161,6 +162,139 @@ __global__ __launch_bounds__(64) void ce_rows_kernel(const float* __restrict__ l
     }
 }
 
+// The same for launches of few rows, whose time is the chains': a workgroup takes two rows, two waves form each row's
+// exponentials chunk by chunk, and a fifth wave adds the chunk before, so a chain waits for its adds alone (in
+// ce_rows_kernel a wave's chain waits while it forms the next exponentials: 33 cycles per column at 1023 x 151936, 2.1 ms;
+// here 1.0 ms). With the chip full of rows the waves that only add cost more than they hide (8184 x 151936: 4.5 ms in
+// ce_rows_kernel, 6.4 here); its two rows per wave reach one wave per SIMD at 2048 rows.
+constexpr int64_t kPipeBelow = 2048;
+constexpr int kPipeRows = 2;
+
+__global__ __launch_bounds__(320) void ce_rows_pipe_kernel(const float* __restrict__ logits,
+                                                           const int64_t* __restrict__ targets, int64_t rows,
+                                                           int64_t vocab, double* __restrict__ row_max,
+                                                           double* __restrict__ row_total,
+                                                           double* __restrict__ row_loss, int* __restrict__ error_flag) {
+    __shared__ __align__(16) double e[2][kPipeRows][kCeLd];
+    __shared__ float best[kPipeRows][2];
+    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kPipeRows;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int lane = static_cast<int>(threadIdx.x) & 63;
+    const int q = wave >> 1, h = wave & 1;  // a producer's row and half of each chunk
+    const bool vec = vocab % 4 == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0;
+    const int64_t row = r0 + q < rows ? r0 + q : rows - 1;  // a missing second row repeats the last one, unused
+    const float* lr = logits + row * vocab;
+    if (wave < 4) {
+        float b = lr[0];
+        int64_t j0 = 0;
+        if (vec) {
+            const float4* l4 = reinterpret_cast<const float4*>(lr);
+            const int64_t n4 = vocab / 4;
+            int64_t k = h * 64 + lane;
+            for (; k + 7 * 128 < n4; k += 8 * 128) {
+                float4 v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = l4[k + u * 128];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    if (v[u].x > b) b = v[u].x;
+                    if (v[u].y > b) b = v[u].y;
+                    if (v[u].z > b) b = v[u].z;
+                    if (v[u].w > b) b = v[u].w;
+                }
+            }
+            for (; k < n4; k += 128) {
+                const float4 v = l4[k];
+                if (v.x > b) b = v.x;
+                if (v.y > b) b = v.y;
+                if (v.z > b) b = v.z;
+                if (v.w > b) b = v.w;
+            }
+            j0 = 4 * n4;
+        }
+        for (int64_t j = j0 + h * 64 + lane; j < vocab; j += 128) {
+            const float v = lr[j];
+            if (v > b) b = v;
+        }
+        for (int off = 32; off >= 1; off >>= 1) {
+            const float o = __shfl_xor(b, off, 64);
+            if (o > b) b = o;
+        }
+        if (lane == 0) best[q][h] = b;
+    }
+    __syncthreads();
+    const auto max_of = [&](int k) {
+        return static_cast<double>(best[k][1] > best[k][0] ? best[k][1] : best[k][0]);
+    };
+    const int64_t chunks = (vocab + kCeChunk - 1) / kCeChunk;
+    if (wave < 4) {
+        const double mx = max_of(q);
+        // columns h 256 + 4 lane .. + 3 of a chunk; past the row's end +0.0 is added, which changes no sum of
+        // exponentials
+        const auto load = [&](int64_t c) {
+            const int64_t j = c * kCeChunk + h * 256 + lane * 4;
+            float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (vec) {
+                if (j < vocab) v = *reinterpret_cast<const float4*>(lr + j);
+            } else {
+                if (j < vocab) v.x = lr[j];
+                if (j + 1 < vocab) v.y = lr[j + 1];
+                if (j + 2 < vocab) v.z = lr[j + 2];
+                if (j + 3 < vocab) v.w = lr[j + 3];
+            }
+            return v;
+        };
+        float4 v = load(0), n1 = load(1);
+        for (int64_t c = 0; c < chunks; ++c) {
+            const float4 n2 = load(c + 2);
+            const int64_t j = c * kCeChunk + h * 256 + lane * 4;
+            double2* out = reinterpret_cast<double2*>(&e[c & 1][q][h * 256 + lane * 4]);
+            out[0] = double2{j < vocab ? dexp(static_cast<double>(v.x) - mx) : 0.0,
+                             j + 1 < vocab ? dexp(static_cast<double>(v.y) - mx) : 0.0};
+            out[1] = double2{j + 2 < vocab ? dexp(static_cast<double>(v.z) - mx) : 0.0,
+                             j + 3 < vocab ? dexp(static_cast<double>(v.w) - mx) : 0.0};
+            lds_barrier();
+            v = n1;
+            n1 = n2;
+        }
+        return;
+    }
+    double total = 0.0;
+    for (int64_t c = 0; c < chunks; ++c) {
+        lds_barrier();  // chunk c is formed; the producers go on to chunk c + 1
+        if (lane >= kPipeRows) continue;
+        const double2* e2 = reinterpret_cast<const double2*>(e[c & 1][lane]);
+        double2 t[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) t[u] = e2[u];
+#pragma unroll 4
+        for (int j = 0; j < kCeChunk / 2; j += 8) {
+            double2 tn[8];
+            const int jn = j + 8 < kCeChunk / 2 ? j + 8 : 0;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) tn[u] = e2[jn + u];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                total += t[u].x;
+                total += t[u].y;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t[u] = tn[u];
+        }
+    }
+    if (lane < kPipeRows && r0 + lane < rows) {
+        const int64_t r = r0 + lane;
+        const double mx = max_of(lane);
+        row_max[r] = mx;
+        row_total[r] = total;
+        const int64_t t = targets[r];
+        if (t >= vocab) *error_flag = 1;
+        row_loss[r] = (t >= 0 && t < vocab) ? mx + dlog(total) - static_cast<double>(logits[r * vocab + t]) : 0.0;
+    }
+}
+
 // dlogits[r][j] = f32((exp(l - max) * (1 / total) - onehot) * scale); zeros for ignored rows. One thread takes four
 // consecutive columns (16-byte loads and stores when the rows allow); the grid strides over rows.
 __device__ __forceinline__ float ce_grad_value(float l, int64_t j, int64_t t, double mx, double inv, double scale) {
@@ -253,8 +387,12 @@ int launch_cross_entropy(const float* logits, const int64_t* targets, float* dlo
     if (rows == 0) return kOk;
     DLLM_REQUIRE(vocab > 0, "cross_entropy needs a non-empty vocabulary");
     DLLM_REQUIRE(ceil_div(rows, kCeRows) <= 0x7fffffffLL, "too many rows");
-    hipLaunchKernelGGL(ce_rows_kernel, dim3(static_cast<unsigned>(ceil_div(rows, kCeRows))), dim3(64), 0, stream,
-                       logits, targets, rows, vocab, row_max, row_total, row_loss, error_flag);
+    if (rows < kPipeBelow)
+        hipLaunchKernelGGL(ce_rows_pipe_kernel, dim3(static_cast<unsigned>(ceil_div(rows, kPipeRows))), dim3(320), 0,
+                           stream, logits, targets, rows, vocab, row_max, row_total, row_loss, error_flag);
+    else
+        hipLaunchKernelGGL(ce_rows_kernel, dim3(static_cast<unsigned>(ceil_div(rows, kCeRows))), dim3(64), 0, stream,
+                           logits, targets, rows, vocab, row_max, row_total, row_loss, error_flag);
     DLLM_TRY(check_launch("cross_entropy rows"));
     const unsigned row_blocks = static_cast<unsigned>(rows < 65535 ? rows : 65535);
     hipLaunchKernelGGL(ce_grad_kernel, dim3(static_cast<unsigned>(ceil_div(vocab, 1024)), row_blocks), dim3(256), 0,
