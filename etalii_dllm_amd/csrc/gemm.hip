@@ -1336,6 +1336,7 @@ int launch_gemm(const GemmCall& g, hipStream_t stream) {
             DLLM_REQUIRE(g.seg == nullptr && g.l0 == 0 && g.l1 % 4 == 0 && g.l1 >= 4 && g.lda >= g.l1,
                          "transposed float A needs a plain reduction over whole 16-byte chunks");
     }
+    if (ak == kAFloatT && chain_linear_fits(g)) return launch_chain_linear(g, stream);
     const SplitPlan split = split_plan(g);
     if (split.rows > 0 && split.rows < g.I) {  // row blocks that share B's split
         for (int64_t i0 = 0; i0 < g.I; i0 += split.rows) {

@@ -26,4 +26,8 @@ SplitPlan split_plan(const GemmCall& g);
 // chains; the tiles of redo->tile_flags are left to the caller. partial: per-window results instead of C.
 int launch_split_gemm(const GemmCall& g, float* partial, hipStream_t stream, SplitRedo* redo);
 
+// Forward matmuls of few outputs, each by its own chain from x and Bt.
+bool chain_linear_fits(const GemmCall& g);
+int launch_chain_linear(const GemmCall& g, hipStream_t stream);
+
 }  // namespace dllm_hip

@@ -856,16 +856,104 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 constexpr int kFixRows = 32;
 constexpr int kFixL = 128;
 
+struct ChainBuffers {
+    // products of l 4 k, 4 k + 1 at 2 k, those of 4 k + 2, 4 k + 3 at kFixL / 2 + 2 k: 16-byte writes of consecutive
+    // lanes are adjacent
+    __attribute__((aligned(16))) double prod[2][kFixRows][kFixL + 2];
+    const float* a[kFixRows];
+    const float* b[kFixRows];
+    int len[kFixRows];
+};
+
+// The serial double sums of a[q][l] b[q][l], l ascending, of the workgroup's kFixRows pairs: the result of pair q in
+// thread 256 + q. Called by all 320 threads once the buffers' pointers and lengths are visible. Loads are 16 bytes: those
+// past a pair's length must read zeros or, for lengths that are multiples of 4, do not happen.
+__device__ __forceinline__ double chains(ChainBuffers& s, int tid) {
+    int longest = 0;
+#pragma unroll 8
+    for (int q = 0; q < kFixRows; ++q) longest = max(longest, s.len[q]);
+    const int chunks = (longest + kFixL - 1) / kFixL;
+    double acc = 0.0;
+    if (tid < 256) {  // wave-uniform
+        constexpr int kN = kFixRows / 8;
+        const int q0 = tid >> 5, lq = (tid & 31) * 4;  // this thread's pairs q0 + 8 k, and its l in a chunk
+        const float *ga[kN], *gb[kN];
+        int len[kN];
+#pragma unroll
+        for (int q = 0; q < kN; ++q) {
+            ga[q] = s.a[q0 + 8 * q] + lq;
+            gb[q] = s.b[q0 + 8 * q] + lq;
+            len[q] = s.len[q0 + 8 * q] - lq;
+        }
+        float4 x0[kN], y0[kN], x1[kN], y1[kN];
+        auto load = [&](float4 (&x)[kN], float4 (&y)[kN], int l) {
+#pragma unroll
+            for (int q = 0; q < kN; ++q) {
+                const bool in = l < len[q];
+                const float4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                x[q] = in ? *reinterpret_cast<const float4*>(ga[q] + l) : zero;
+                y[q] = in ? *reinterpret_cast<const float4*>(gb[q] + l) : zero;
+            }
+        };
+        auto form = [&](const float4 (&x)[kN], const float4 (&y)[kN], int c) {
+#pragma unroll
+            for (int q = 0; q < kN; ++q) {
+                double* d = &s.prod[c & 1][q0 + 8 * q][lq / 2];
+                *reinterpret_cast<double2*>(d) = double2{static_cast<double>(x[q].x) * static_cast<double>(y[q].x),
+                                                         static_cast<double>(x[q].y) * static_cast<double>(y[q].y)};
+                *reinterpret_cast<double2*>(d + kFixL / 2) =
+                    double2{static_cast<double>(x[q].z) * static_cast<double>(y[q].z),
+                            static_cast<double>(x[q].w) * static_cast<double>(y[q].w)};
+            }
+        };
+        load(x0, y0, 0);
+        load(x1, y1, kFixL);
+        for (int c = 0; c < chunks; c += 2) {
+            form(x0, y0, c);
+            load(x0, y0, (c + 2) * kFixL);
+            lds_barrier();
+            if (c + 1 >= chunks) break;
+            form(x1, y1, c + 1);
+            load(x1, y1, (c + 3) * kFixL);
+            lds_barrier();
+        }
+        return acc;
+    }
+    for (int c = 0; c < chunks; ++c) {
+        lds_barrier();  // chunk c is formed; the producers go on to chunk c + 1
+        if (tid - 256 < kFixRows) {  // past a pair's length the products are +0, which change no sum
+            const double2* lo = reinterpret_cast<const double2*>(s.prod[c & 1][tid - 256]);
+            const double2* hi = lo + kFixL / 4;
+            double2 t[8];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) t[2 * u] = lo[u], t[2 * u + 1] = hi[u];
+#pragma unroll
+            for (int e = 0; e < kFixL / 4; e += 4) {  // 16 l
+                double2 tn[8];
+                const int en = e + 4 < kFixL / 4 ? e + 4 : 0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) tn[2 * u] = lo[en + u], tn[2 * u + 1] = hi[en + u];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    acc = acc + t[u].x;
+                    acc = acc + t[u].y;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) t[u] = tn[u];
+            }
+        }
+    }
+    return acc;
+}
+
 template <bool kSeg>
 __global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2))) void split_fix_kernel(SplitParams p) {
-    __shared__ double prod[2][kFixRows][kFixL + 2];
-    __shared__ const float* pa[kFixRows];
-    __shared__ const float* pb[kFixRows];
-    __shared__ int plen[kFixRows];
+    __shared__ ChainBuffers s_mem;
     const uint32_t n = *p.count < p.list_cap ? *p.count : p.list_cap;
     const int tid = static_cast<int>(threadIdx.x);
-    const bool producer = tid < 256;                             // wave-uniform
-    const bool owner = tid >= 256 && tid - 256 < kFixRows;       // the lanes that add
+    const bool owner = tid >= 256 && tid - 256 < kFixRows;  // the lanes that add
     const int row = owner ? tid - 256 : 0;
     const bool sequence = kSeg && !p.partial;
     for (uint32_t k0 = blockIdx.x * kFixRows; k0 < n; k0 += gridDim.x * kFixRows) {
@@ -881,84 +969,13 @@ __global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2))) void s
         __syncthreads();  // the pairs before are done
         if (owner) {
             const Window w = window_of(p, s);
-            pa[row] = p.a.rows_contiguous ? p.a.t + (i * p.stages + w.stage0) * kStageL : p.a.src + i * p.a.ld;
-            pb[row] = p.b.rows_contiguous ? p.b.t + (j * p.stages + w.stage0) * kStageL : p.b.src + j * p.b.ld;
-            plen[row] = valid ? static_cast<int>(w.l1 - w.l0) : 0;
+            s_mem.a[row] = p.a.rows_contiguous ? p.a.t + (i * p.stages + w.stage0) * kStageL : p.a.src + i * p.a.ld;
+            s_mem.b[row] = p.b.rows_contiguous ? p.b.t + (j * p.stages + w.stage0) * kStageL : p.b.src + j * p.b.ld;
+            s_mem.len[row] = valid ? static_cast<int>(w.l1 - w.l0) : 0;
         }
         __syncthreads();
-        int longest = 0;
-#pragma unroll 8
-        for (int q = 0; q < kFixRows; ++q) longest = max(longest, plen[q]);
-        const int chunks = (longest + kFixL - 1) / kFixL;
-        if (producer) {
-            constexpr int kN = kFixRows / 8;
-            const int q0 = tid >> 5, lq = (tid & 31) * 4;  // this thread's pairs q0 + 8 k, and its l in a chunk
-            const float *ga[kN], *gb[kN];
-            int len[kN];
-#pragma unroll
-            for (int q = 0; q < kN; ++q) {
-                ga[q] = pa[q0 + 8 * q] + lq;
-                gb[q] = pb[q0 + 8 * q] + lq;
-                len[q] = plen[q0 + 8 * q] - lq;
-            }
-            float4 x0[kN], y0[kN], x1[kN], y1[kN];
-            // A 16-byte load past a window's end reads the zeros of the transposed copy; a row-major operand's
-            // reduction is a multiple of 4 long.
-            auto load = [&](float4 (&x)[kN], float4 (&y)[kN], int l) {
-#pragma unroll
-                for (int q = 0; q < kN; ++q) {
-                    const bool in = l < len[q];
-                    const float4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-                    x[q] = in ? *reinterpret_cast<const float4*>(ga[q] + l) : zero;
-                    y[q] = in ? *reinterpret_cast<const float4*>(gb[q] + l) : zero;
-                }
-            };
-            auto form = [&](const float4 (&x)[kN], const float4 (&y)[kN], int c) {
-#pragma unroll
-                for (int q = 0; q < kN; ++q) {
-                    double* d = &prod[c & 1][q0 + 8 * q][lq];
-                    d[0] = static_cast<double>(x[q].x) * static_cast<double>(y[q].x);
-                    d[1] = static_cast<double>(x[q].y) * static_cast<double>(y[q].y);
-                    d[2] = static_cast<double>(x[q].z) * static_cast<double>(y[q].z);
-                    d[3] = static_cast<double>(x[q].w) * static_cast<double>(y[q].w);
-                }
-            };
-            load(x0, y0, 0);
-            load(x1, y1, kFixL);
-            for (int c = 0; c < chunks; c += 2) {
-                form(x0, y0, c);
-                load(x0, y0, (c + 2) * kFixL);
-                lds_barrier();
-                if (c + 1 >= chunks) break;
-                form(x1, y1, c + 1);
-                load(x1, y1, (c + 3) * kFixL);
-                lds_barrier();
-            }
-            continue;
-        }
-        double acc = 0.0;
-        for (int c = 0; c < chunks; ++c) {
-            lds_barrier();  // chunk c is formed; the producers go on to chunk c + 1
-            if (owner) {    // past a pair's length the products are +0, which change no sum
-                const double* d = prod[c & 1][row];
-                double t[16];
-#pragma unroll
-                for (int u = 0; u < 16; ++u) t[u] = d[u];
-#pragma unroll
-                for (int e = 0; e < kFixL; e += 16) {
-                    double tn[16];
-                    const int en = e + 16 < kFixL ? e + 16 : 0;
-#pragma unroll
-                    for (int u = 0; u < 16; ++u) tn[u] = d[en + u];
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int u = 0; u < 16; ++u) acc = acc + t[u];
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int u = 0; u < 16; ++u) t[u] = tn[u];
-                }
-            }
-        }
+        // past a window's end the transposed copy holds zeros; a row-major operand's reduction is a multiple of 4
+        double acc = chains(s_mem, tid);
         if (!owner || !valid) continue;
         if constexpr (!kSeg) {
             if (p.bias) acc += static_cast<double>(p.bias[j]);
@@ -979,6 +996,35 @@ __global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2))) void s
                 p.partial[(static_cast<int64_t>(s) * p.I + i) * p.J + j] = v;
         }
     }
+}
+
+// A forward matmul of few outputs (a token or a few through a projection): every output's chain as above, straight from
+// x and the weight's rows, 32 outputs per workgroup (rows of a token side by side, so a weight row is read once from
+// memory). The time is a read of the weight and one chain. 1 x 896 x 4864: the transpose of the weight and 32 x 32 tiles
+// took 22.8 us, this takes 11.8.
+__global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2))) void chain_linear_kernel(
+    const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw, const float* __restrict__ bias,
+    const float* __restrict__ addsrc, int64_t ld_add, float* __restrict__ out, int64_t ldc, int64_t rows, int64_t outs,
+    int len) {
+    __shared__ ChainBuffers s_mem;
+    const int tid = static_cast<int>(threadIdx.x);
+    const bool owner = tid >= 256 && tid - 256 < kFixRows;
+    const int q = owner ? tid - 256 : 0;
+    const int64_t k = static_cast<int64_t>(blockIdx.x) * kFixRows + q;
+    const bool valid = k < rows * outs;
+    const int64_t i = valid ? k % rows : 0, j = valid ? k / rows : 0;
+    if (owner) {
+        s_mem.a[q] = x + i * ldx;
+        s_mem.b[q] = w + j * ldw;
+        s_mem.len[q] = valid ? len : 0;
+    }
+    __syncthreads();
+    double acc = chains(s_mem, tid);
+    if (!owner || !valid) return;
+    if (bias) acc += static_cast<double>(bias[j]);
+    float v = static_cast<float>(acc);
+    if (addsrc) v = addsrc[i * ld_add + j] + v;
+    out[i * ldc + j] = v;
 }
 
 // Windows in sequence: each slot's output from the sum before its first undecided window and the results after it.
@@ -1102,6 +1148,26 @@ SplitPlan split_plan(const GemmCall& g) {
             return plan;
         }
     return plan;
+}
+
+// Few outputs: 256 workgroups (8192 outputs) side by side take 10.7 ns per l and 2 us, the tiled matmul 13.6 ns per l and,
+// where it has to be made, the weight's transpose at about 2.5 TB/s. 1 x 896 x 4864: 11.8 us against 22.8; 2 x 896 x 4864:
+// 20.9 against 22.8; 4 x 896 x 4864: 30.1 against 22.9 (not taken); 4 x 8960 x 1536: 78 against 122; 1 x 2048 x 50304:
+// 160 against 476.
+bool chain_linear_fits(const GemmCall& g) {
+    if (g.a_kind != 2 || g.Bt == nullptr || g.seg != nullptr || g.l0 != 0 || g.l1 <= 0 || g.l1 >= (1 << 30)) return false;
+    if (g.I > 64) return false;
+    const double L = static_cast<double>(g.l1);
+    const double transpose = g.bt_transpose ? 8.0 * L * static_cast<double>(g.J) / 2.5e12 : 0.0;
+    return static_cast<double>(ceil_div(g.I * g.J, 256 * kFixRows)) * L * 10.7e-9 + 2e-6 < L * 13.6e-9 + transpose;
+}
+
+int launch_chain_linear(const GemmCall& g, hipStream_t stream) {
+    const int64_t pairs = g.I * g.J;
+    hipLaunchKernelGGL(chain_linear_kernel, dim3(static_cast<unsigned>(ceil_div(pairs, kFixRows))), dim3(320), 0, stream,
+                       g.Af, g.lda, g.Bt, g.ldbt, g.bias, g.addsrc, g.ld_add, g.C, g.ldc, g.I, g.J,
+                       static_cast<int>(g.l1));
+    return check_launch("chain linear");
 }
 
 int launch_split_gemm(const GemmCall& g, float* partial, hipStream_t stream, SplitRedo* redo) {

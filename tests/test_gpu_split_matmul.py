@@ -80,3 +80,13 @@ def test_linear_backward(K, kind, rows, inf, outf):
     cols = np.array([0, 11, 12, outf - 1])
     ora = O.oracle_kernels().linear_backward(x, w[cols].copy(), dy[:, cols].copy())
     assert_same(dw[cols], ora[1], "oracle dw")
+
+
+@pytest.mark.parametrize("kind", ["gauss", "wide", "special"])
+@pytest.mark.parametrize("rows,inf,outf", [(1, 132, 36), (1, 896, 4864), (2, 1028, 4092), (5, 252, 1000), (1, 4, 40)])
+def test_linear_of_few_rows(K, kind, rows, inf, outf):
+    """A token or a few through a projection: every output by its own chain."""
+    x, w = operand("gauss", 7, rows, inf), operand(kind if inf > 13 and outf > 200 else "gauss", 8, outf, inf)
+    b = operand("gauss", 9, 1, outf)[0]
+    assert_same(K.linear(x, w, b), O.oracle_kernels().linear(x, w, b), "linear")
+    assert_same(K.linear(x, w), K.linear(np.repeat(x, 80, axis=0), w)[::80], "the same rows in a larger call")
