@@ -692,32 +692,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
         if (use6) {
-            // The sixth digit's products with the first, (1, 6) and (6, 1), into the last accumulator: the same steps with
-            // two digits of each block, through the same buffers.
-            auto issue6 = [&](int64_t c) {
+            // The sixth digit's products with the first, (1, 6) and (6, 1), into the last accumulator: two digits of each
+            // block, kBatch steps to a barrier, the next ones on their way to the other half of the ring.
+            constexpr int kBatch = 3;
+            static_assert(2 * kBatch * 8 <= kRing * kCopies, "two batches of 8 KB steps in the ring");
+            int8_t* const half0 = &ring[0][0];
+            auto issue6 = [&](int64_t c) {  // past the last step: the last one again, never used
+                const bool isa = wave < 2;  // this wave's block: A's two, then B's
+                const int64_t last = (isa ? p.a.blocks : p.b.blocks) - 1;
+                const int64_t want = isa ? i_blk / 32 + wave : j_blk / 32 + wave - 2;
+                const int64_t row = (want < last ? want : last) * p.stages * 2 + step0;
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const int blk = wave;  // A's two, then B's
-                    const bool isa = blk < 2;
-                    const int64_t last = (isa ? p.a.blocks : p.b.blocks) - 1;
-                    const int64_t want = isa ? i_blk / 32 + blk : j_blk / 32 + blk - 2;
-                    const int64_t at = (want < last ? want : last) * p.stages * 2 + step0 + c;
-                    const int8_t* from = t == 0 ? (isa ? p.a.digits : p.b.digits) + at * kStepBytes
-                                                : (isa ? p.a.digits6 : p.b.digits6) + at * kFragment;
-                    copy16_to_lds_s(from, voff, &ring[c % 2][(2 * blk + t) * kFragment]);
+                for (int t = 0; t < 2 * kBatch; ++t) {
+                    const int64_t at = row + (c + t / 2 < steps ? c + t / 2 : steps - 1);
+                    const int8_t* from = t % 2 == 0 ? (isa ? p.a.digits : p.b.digits) + at * kStepBytes
+                                                    : (isa ? p.a.digits6 : p.b.digits6) + at * kFragment;
+                    copy16_to_lds_s(from, voff, half0 + (c / kBatch % 2 * kBatch * 8 + t / 2 * 8 + 2 * wave + t % 2) *
+                                                            kFragment);
                 }
             };
             if (steps > 0) issue6(0);
-            for (int64_t c = 0; c < steps; ++c) {
+            for (int64_t c = 0; c < steps; c += kBatch) {
                 asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                if (c + 1 < steps) issue6(c + 1);
-                const int8_t* mem = ring[c % 2] + lane * 16;
-                const v4i a1 = *reinterpret_cast<const v4i*>(mem + wi * 2 * kFragment);
-                const v4i a6 = *reinterpret_cast<const v4i*>(mem + (wi * 2 + 1) * kFragment);
-                const v4i b1 = *reinterpret_cast<const v4i*>(mem + (2 + wj) * 2 * kFragment);
-                const v4i b6 = *reinterpret_cast<const v4i*>(mem + ((2 + wj) * 2 + 1) * kFragment);
-                acc[kOrders - 1] = mfma_i8(a1, b6, acc[kOrders - 1]);
-                acc[kOrders - 1] = mfma_i8(a6, b1, acc[kOrders - 1]);
+                if (c + kBatch < steps) issue6(c + kBatch);
+#pragma unroll
+                for (int t = 0; t < kBatch; ++t) {
+                    if (c + t >= steps) break;
+                    const int8_t* mem = half0 + (c / kBatch % 2 * kBatch * 8 + t * 8) * kFragment + lane * 16;
+                    const v4i a1 = *reinterpret_cast<const v4i*>(mem + wi * 2 * kFragment);
+                    const v4i a6 = *reinterpret_cast<const v4i*>(mem + (wi * 2 + 1) * kFragment);
+                    const v4i b1 = *reinterpret_cast<const v4i*>(mem + (2 + wj) * 2 * kFragment);
+                    const v4i b6 = *reinterpret_cast<const v4i*>(mem + ((2 + wj) * 2 + 1) * kFragment);
+                    acc[kOrders - 1] = mfma_i8(a1, b6, acc[kOrders - 1]);
+                    acc[kOrders - 1] = mfma_i8(a6, b1, acc[kOrders - 1]);
+                }
             }
         }
 
