@@ -6,20 +6,24 @@
 // that bound leaves the rounding open.
 //
 //   Split. Each row of an operand (A's i or B's j, over the reduction l of one window) is scaled by a power of two to
-//   40-bit integers and cut into five signed base-256 digits, d_1 (high) to d_5. a = sum_p d_p 256^(5-p) exactly for
-//   floats down to 2^-16 of the row's largest; below that a is rounded, by at most half a unit.
-//   Products. sum_l a_l b_l = sum over (p, q) of 256^(10-p-q) sum_l d_p(a_l) d_q(b_l). The 19 pairs with p + q <= 7
-//   are int8 matrix products, exact in int32 (a window's length is limited to 24576, so 5 pairs x 2^14 x L < 2^31);
-//   pairs of equal p + q share an accumulator.
+//   48-bit integers and cut into six signed base-256 digits, d_1 (high) to d_6. a = sum_p d_p 256^(6-p) exactly for floats
+//   down to 2^-24 of the row's largest; below that a is rounded, by at most half a unit.
+//   Products. sum_l a_l b_l is a sum over digit pairs (p, q), each a matrix product of int8. The 19 pairs of the first five
+//   digits with p + q <= 7 are formed, exact in int32 (a window's length is limited so that 6 pairs x 2^14 x L < 2^31); pairs
+//   of equal p + q share an accumulator. The sixth digit is nearly always zero; a tile for which its norm matters adds the
+//   pairs (1, 6) and (6, 1).
 //   Bound. With N = ||a||_2 of a row (and N_p of its digits, r of its rounding), Cauchy-Schwarz bounds what is left
 //   out: 2^16 (N_3a N_5b + N_4a N_4b + N_5a N_3b) + 2^8 (N_4a N_5b + N_5a N_4b) + N_5a N_5b + r_a N_b + N_a r_b + r_a r_b.
 //   The chain itself is off by at most 2^-53 sum_k |s_k| over its partial sums s_k; with the integer partial sum S_c
 //   known at every 128th l, |s_k| <= |S_c| + (the norms over the 128 values in between), whose sum over all chunks is
 //   at most 128 N_a N_b (Cauchy-Schwarz over the chunks).
 //   Decision. When the integer sum plus and minus the bound round to the same float, the chain rounds to it too.
-//   Otherwise the output goes to a list, and split_fix_kernel computes its chain. On Gaussian operands that is about
-//   one output in 2000. A tile of which more than one in 32 would go there (rows of very wide dynamic range, infinities,
-//   NaNs) is flagged and recomputed whole by the FP64 matmul.
+//   Otherwise the output goes to a list, and split_fix_kernel computes its chain: one output in 2500 on Gaussian operands
+//   at L = 1536, one in 260 at 8192 with rows and columns of unequal size. A tile of which more than one in 64 would go
+//   there (rows of very wide dynamic range, infinities, NaNs) is flagged and recomputed whole by the FP64 matmul.
+//   Measured: 1023 x 8960 x 1536 in 265 us of 380 for the call, against 600 in FP64; 8192 x 1536 x 8960 in 1.67 ms (135
+//   TFLOP/s), with splitting and recomputation 2.5, against 3.3. The matrix cores' power bounds it: random digits hold the
+//   clock at 1.7 GHz with them busy throughout, 181 TFLOP/s.
 #include <algorithm>
 
 #include "common.h"
@@ -100,6 +104,7 @@ struct SplitParams {
     uint64_t* slots;
     float* slot_values;  // [slot][1 + nseg]
     uint32_t slot_cap;
+    uint32_t* stat;  // flagged tiles of the caller's (null: none kept)
 };
 
 struct Window {
@@ -837,7 +842,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     if (tid == 0) {
         *flag = heavy ? 1 : 0;
-        if (heavy) atomicAdd(&p.count[1], 1u);
+        if (heavy) {
+            atomicAdd(&p.count[1], 1u);
+            if (p.stat) atomicAdd(p.stat, 1u);
+        }
     }
     if (heavy) return;
     float* out = p.partial ? p.partial + static_cast<int64_t>(blockIdx.y) * p.I * p.J : p.C;
@@ -1222,6 +1230,7 @@ int launch_split_gemm(const GemmCall& g, float* partial, hipStream_t stream, Spl
     p.seg_weight = g.seg_weight;
     p.seg_rowscale = g.seg_rowscale;
     p.partial = partial;
+    p.stat = g.split_stat;
     // a shared operand that the call before left in the scratch is not split again
     const bool a_ready = g.split_ready && g.split_share == 1, b_ready = g.split_ready && g.split_share == 2;
     const int64_t per = 32 * l.nseg * static_cast<int64_t>(sizeof(RowMeta) / 16);

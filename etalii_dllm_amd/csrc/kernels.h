@@ -60,6 +60,8 @@ struct GemmCall {
     // the call before, of the same share, reduction and windows, left it in the scratch.
     int split_share = 0;
     bool split_ready = false;
+    uint32_t* split_stat = nullptr;  // optional device counter: the tiles that the path hands back to FP64 are added
+    int split_site = -1;             // the caller's own number of the call
 };
 // The rows of a block of the call on the int8 path: I when it runs there whole, 0 when it does not run there.
 int64_t gemm_split_rows(const GemmCall& g);

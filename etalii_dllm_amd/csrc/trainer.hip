@@ -27,6 +27,7 @@
 #include <map>
 #include <memory>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "attn_step.h"
@@ -210,6 +211,15 @@ struct dllm_hip_trainer {
     int64_t gemm_part_cap = 0;  // floats: per-window partials of the layer weight gradients
     char* split_mem[2] = {nullptr, nullptr};  // the int8 matmuls' scratch: the step's stream, the side stream
     size_t split_cap[2] = {0, 0};
+    // How the int8 path fares at each matmul of the step (3 x weight + forward, input gradient, weight gradient): the tiles
+    // it handed back in the step (device) of those it ran, and for how many steps more the matmul runs in FP64. Operands
+    // of very wide range (gradients of a batch learnt by heart) hand most tiles back, at the cost of both paths.
+    static constexpr int kSplitRest = 32;
+    uint32_t* split_stat = nullptr;
+    std::vector<uint32_t> split_handed;
+    std::vector<int64_t> split_tiles;
+    std::vector<int> split_rest;
+    std::unordered_map<int64_t, int> tensor_at;  // by offset in the arenas
     // routed experts: E experts, K per token, EI expert intermediate size; shared buffers of the grouped rows
     int64_t E = 0, K = 0, EI = 0, RK = 0;
     float *xg = nullptr, *dyg = nullptr, *dxg = nullptr, *dweights = nullptr, *dlogits_r = nullptr, *dprob = nullptr,
@@ -632,6 +642,15 @@ struct dllm_hip_trainer {
             split_cap[k] = std::min(split_bytes(k == 1), kSplitMax);
             if (split_cap[k] > 0) DLLM_TRY(make(&split_mem[k], split_cap[k]));
         }
+        if (split_cap[0] > 0) {
+            const size_t sites = 3 * tensors.size();
+            DLLM_TRY(make(&split_stat, sites));
+            DLLM_TRY(check_hip(hipMemset(split_stat, 0, sites * sizeof(uint32_t)), "memset"));
+            split_handed.assign(sites, 0);
+            split_tiles.assign(sites, 0);
+            split_rest.assign(sites, 0);
+            for (size_t i = 0; i < tensors.size(); ++i) tensor_at[tensors[i].offset] = static_cast<int>(i);
+        }
         DLLM_TRY(make(&emb_rows, R * H));
         DLLM_TRY(make(&inv_rms, R * std::max<int64_t>(heads, 1)));
         DLLM_TRY(make(&inv_mlp, R));
@@ -931,13 +950,32 @@ struct dllm_hip_trainer {
     // The call with the int8 path's scratch of its stream.
     GemmCall with_split(const GemmCall& g, hipStream_t s) const {
         GemmCall c = g;
+        if (split_stat != nullptr && g.split_site >= 0) {
+            if (split_rest[static_cast<size_t>(g.split_site)] > 0) return c;
+            c.split_stat = split_stat + g.split_site;
+        }
         const int k = side_on && s == side ? 1 : 0;
         c.split_scratch = split_mem[k];
         c.split_cap = split_cap[k];
         return c;
     }
 
+    // After a step's synchronisation: matmuls that handed back more than a third of their tiles rest.
+    int split_review(hipStream_t s) {
+        if (split_stat == nullptr) return kOk;
+        for (size_t i = 0; i < split_handed.size(); ++i) {
+            if (split_rest[i] > 0) --split_rest[i];
+            if (3 * static_cast<int64_t>(split_handed[i]) > split_tiles[i]) split_rest[i] = kSplitRest;
+            split_tiles[i] = 0;
+        }
+        return check_hip(hipMemsetAsync(split_stat, 0, split_handed.size() * sizeof(uint32_t), s), "memset");
+    }
+
     int gemm(const GemmCall& g, hipStream_t s) {
+        if (split_stat != nullptr && g.split_site >= 0 && gemm_split_rows(with_split(g, s)) > 0) {
+            const int64_t tiles = ceil_div(g.I, 64) * ceil_div(g.J, 64);  // of each window, where they run in parallel
+            split_tiles[static_cast<size_t>(g.split_site)] += tiles * (g.seg && tiles < 2048 ? g.nseg : 1);
+        }
         if (!profiling) return launch_gemm(with_split(g, s), s);
         DLLM_TRY(profile_begin(s));
         DLLM_TRY(launch_gemm(with_split(g, s), s));
@@ -1127,6 +1165,7 @@ struct dllm_hip_trainer {
         g.ldb = N;
         g.Bt = P(w_id);
         g.ldbt = K;
+        g.split_site = 3 * w_id;
         g.C = out;
         g.ldc = N;
         g.I = R;
@@ -1156,6 +1195,7 @@ struct dllm_hip_trainer {
         g.ldb = t.cols;
         g.Bt = WT(w_id);
         g.ldbt = t.rows;
+        g.split_site = 3 * w_id + 1;
         g.C = out;
         g.ldc = t.cols;
         g.I = R;
@@ -1196,6 +1236,8 @@ struct dllm_hip_trainer {
         g.nseg = nseg;
         g.l0 = 0;
         g.l1 = seg ? rows : seg_host.back();
+        const auto at = tensor_at.find(out - grads.as<float>());
+        if (at != tensor_at.end()) g.split_site = 3 * at->second + 2;
         if (!seg)
             for (size_t w = 0; w + 1 < seg_host.size(); ++w)
                 g.seg_max = std::max(g.seg_max, seg_host[w + 1] - seg_host[w]);
@@ -2037,7 +2079,11 @@ struct dllm_hip_trainer {
         if (E > 0)
             DLLM_TRY(check_hip(hipMemcpyAsync(&route_flag, route_err, sizeof route_flag, hipMemcpyDeviceToHost, s),
                                "download"));
+        if (split_stat != nullptr)
+            DLLM_TRY(check_hip(hipMemcpyAsync(split_handed.data(), split_stat, split_handed.size() * sizeof(uint32_t),
+                                              hipMemcpyDeviceToHost, s), "download"));
         DLLM_TRY(check_hip(hipStreamSynchronize(s), "step"));
+        DLLM_TRY(split_review(s));
         DLLM_REQUIRE(flag == 0, "target out of range");
         DLLM_REQUIRE(route_flag == 0, "routing produced an expert out of range");
         window_losses = lw;
