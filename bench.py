@@ -629,6 +629,7 @@ def main() -> int:
                    "layers": cfg["layers"], "hidden": cfg["hidden"], "vocab": cfg["vocab"]},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS if achieved else None, "traffic": traffic,
+                     "note": "peak is FP64's; large matmuls run on the int8 matrix cores (19 exact digit products each)",
                      "kernel": "gemm_mfma_kernel (FP64 MFMA matmul, every launch of the matmul-timing steps)",
                      "timing_steps": roofline_steps,
                      "step_fraction_of_peak": matmul_flops_per_step(cfg) / (ms_per_step * 1e9) / FP64_PEAK_TFLOPS},
