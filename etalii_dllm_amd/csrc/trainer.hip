@@ -638,19 +638,6 @@ struct dllm_hip_trainer {
             gemm_part_cap = W_max * H * std::max<int64_t>({QD, KVD, I, EI, E});
             DLLM_TRY(make(&gemm_part, gemm_part_cap));
         }
-        for (int k = 0; k < 2; ++k) {
-            split_cap[k] = std::min(split_bytes(k == 1), kSplitMax);
-            if (split_cap[k] > 0) DLLM_TRY(make(&split_mem[k], split_cap[k]));
-        }
-        if (split_cap[0] > 0) {
-            const size_t sites = 3 * tensors.size();
-            DLLM_TRY(make(&split_stat, sites));
-            DLLM_TRY(check_hip(hipMemset(split_stat, 0, sites * sizeof(uint32_t)), "memset"));
-            split_handed.assign(sites, 0);
-            split_tiles.assign(sites, 0);
-            split_rest.assign(sites, 0);
-            for (size_t i = 0; i < tensors.size(); ++i) tensor_at[tensors[i].offset] = static_cast<int>(i);
-        }
         DLLM_TRY(make(&emb_rows, R * H));
         DLLM_TRY(make(&inv_rms, R * std::max<int64_t>(heads, 1)));
         DLLM_TRY(make(&inv_mlp, R));
@@ -945,6 +932,27 @@ struct dllm_hip_trainer {
             most = std::max(most, split_gemm_bytes(dw));
         }
         return most;
+    }
+
+    // The int8 path's scratch, after everything else: of the memory that is left at most half for each stream, 2 GiB kept
+    // free (a trainer that fits without it is made without it; its matmuls then run in smaller row blocks or in FP64).
+    int split_setup() {
+        size_t free_bytes = 0, total_bytes = 0;
+        DLLM_TRY(check_hip(hipMemGetInfo(&free_bytes, &total_bytes), "hipMemGetInfo"));
+        const size_t keep = size_t{2} << 30, left = free_bytes > keep ? (free_bytes - keep) / 2 : 0;
+        for (int k = 0; k < 2; ++k) {
+            split_cap[k] = std::min({split_bytes(k == 1), kSplitMax, left});
+            if (split_cap[k] > 0) DLLM_TRY(make(&split_mem[k], split_cap[k]));
+        }
+        if (split_cap[0] == 0) return kOk;
+        const size_t sites = 3 * tensors.size();
+        DLLM_TRY(make(&split_stat, sites));
+        DLLM_TRY(check_hip(hipMemset(split_stat, 0, sites * sizeof(uint32_t)), "memset"));
+        split_handed.assign(sites, 0);
+        split_tiles.assign(sites, 0);
+        split_rest.assign(sites, 0);
+        for (size_t i = 0; i < tensors.size(); ++i) tensor_at[tensors[i].offset] = static_cast<int>(i);
+        return kOk;
     }
 
     // The call with the int8 path's scratch of its stream.
@@ -2501,6 +2509,7 @@ int dllm_hip_trainer_create_lora(const dllm_hip_decoder_config* config, const dl
                            "upload"));
         DLLM_TRY(t->setup_fold());
     }
+    DLLM_TRY(t->split_setup());
     *out = t.release();
     return kOk;
 }
