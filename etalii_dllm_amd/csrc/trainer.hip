@@ -940,10 +940,9 @@ struct dllm_hip_trainer {
         size_t free_bytes = 0, total_bytes = 0;
         DLLM_TRY(check_hip(hipMemGetInfo(&free_bytes, &total_bytes), "hipMemGetInfo"));
         const size_t keep = size_t{2} << 30, left = free_bytes > keep ? (free_bytes - keep) / 2 : 0;
-        for (int k = 0; k < 2; ++k) {
-            split_cap[k] = std::min({split_bytes(k == 1), kSplitMax, left});
-            if (split_cap[k] > 0) DLLM_TRY(make(&split_mem[k], split_cap[k]));
-        }
+        // the step's stream only: what runs on the side stream, the layers' weight gradients, stays on FP64
+        split_cap[0] = std::min({split_bytes(false), kSplitMax, left});
+        if (split_cap[0] > 0) DLLM_TRY(make(&split_mem[0], split_cap[0]));
         if (split_cap[0] == 0) return kOk;
         const size_t sites = 3 * tensors.size();
         DLLM_TRY(make(&split_stat, sites));
