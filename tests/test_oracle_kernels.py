@@ -268,6 +268,7 @@ def test_sum_squares_is_the_serial_double_chain():
     assert O.oracle_kernels().sum_squares(g) == acc
 
 
+@needs_ref
 @pytest.mark.parametrize("name", sorted(O.q8_0_cases()))
 def test_quantize_q8_0_matches_reference(name):
     x = O.q8_0_cases()[name]
