@@ -61,6 +61,18 @@ def build(verbose: bool = False) -> Path:
     return LIBRARY
 
 
+def build_test_calls() -> None:
+    """tests/native: host code that hands the library's internal matmul call to the tests (g++, linked to the library)."""
+    native = ROOT / "tests" / "native"
+    rocm = Path(HIPCC).resolve().parents[1]
+    cmd = ["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", f"-I{rocm / 'include'}", f"-I{CSRC}",
+           str(native / "matmul_calls.cpp"), "-o", str(native / "libmatmul_calls.so"), f"-L{PACKAGE}", "-ldllm_hip",
+           f"-Wl,-rpath,$ORIGIN/../../{PACKAGE.name}"]
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"g++ failed for matmul_calls.cpp:\n{result.stderr[-4000:]}")
+
+
 def build_oracle() -> None:
     """The CPU checker (oracle/liboracle.so) and, where the reference checkout exists, oracle/_ref."""
     subprocess.run(["make", "-C", str(ROOT / "oracle")], check=True, capture_output=True)
@@ -68,4 +80,5 @@ def build_oracle() -> None:
 
 if __name__ == "__main__":
     build(verbose=True)
+    build_test_calls()
     build_oracle()

@@ -1059,9 +1059,27 @@ GemmParams params_of(const GemmCall& g) {
                       g.seg_rowscale, g.ld_addrow ? g.ld_addrow : g.I, nullptr};
 }
 
+// Few outputs go to the chain kernel first (chain_linear_fits: as launch_gemm asks).
+bool takes_chains(const GemmCall& g) { return g.a_kind == kAFloatT && !g.split_block && chain_linear_fits(g); }
+
 }  // namespace
 
-int64_t gemm_split_rows(const GemmCall& g) { return mfma_shape(g) ? split_plan(g).rows : 0; }
+int64_t gemm_split_rows(const GemmCall& g) { return mfma_shape(g) && !takes_chains(g) ? split_plan(g).rows : 0; }
+
+GemmCall gemm_split_block(const GemmCall& g, int64_t rows, int64_t i0) {
+    GemmCall b = g;
+    b.I = std::min(rows, g.I - i0);
+    b.Af = g.a_kind == kAFloatT ? g.Af + i0 * g.lda : g.Af + i0;
+    b.C = g.C + i0 * g.ldc;
+    if (g.addsrc) b.addsrc = g.addsrc + i0 * g.ld_add;
+    if (g.seg_addrow) b.seg_addrow = g.seg_addrow + i0;
+    b.ld_addrow = g.ld_addrow ? g.ld_addrow : g.I;
+    if (g.seg_rowscale) b.seg_rowscale = g.seg_rowscale + i0;
+    b.split_block = true;
+    b.split_share = 2;
+    b.split_ready = i0 > 0;
+    return b;
+}
 
 bool gemm_mfma_shape(const GemmCall& g) { return g.a_kind != kADouble && mfma_shape(g); }
 
@@ -1336,22 +1354,10 @@ int launch_gemm(const GemmCall& g, hipStream_t stream) {
             DLLM_REQUIRE(g.seg == nullptr && g.l0 == 0 && g.l1 % 4 == 0 && g.l1 >= 4 && g.lda >= g.l1,
                          "transposed float A needs a plain reduction over whole 16-byte chunks");
     }
-    if (ak == kAFloatT && chain_linear_fits(g)) return launch_chain_linear(g, stream);
+    if (takes_chains(g)) return launch_chain_linear(g, stream);
     const SplitPlan split = split_plan(g);
-    if (split.rows > 0 && split.rows < g.I) {  // row blocks that share B's split
-        for (int64_t i0 = 0; i0 < g.I; i0 += split.rows) {
-            GemmCall b = g;
-            b.I = std::min(split.rows, g.I - i0);
-            b.Af = ak == kAFloatT ? g.Af + i0 * g.lda : g.Af + i0;
-            b.C = g.C + i0 * g.ldc;
-            if (g.addsrc) b.addsrc = g.addsrc + i0 * g.ld_add;
-            if (g.seg_addrow) b.seg_addrow = g.seg_addrow + i0;
-            b.ld_addrow = g.ld_addrow ? g.ld_addrow : g.I;
-            if (g.seg_rowscale) b.seg_rowscale = g.seg_rowscale + i0;
-            b.split_share = 2;
-            b.split_ready = i0 > 0 && gemm_split_rows(b) == b.I;
-            DLLM_TRY(launch_gemm(b, stream));
-        }
+    if (split.rows > 0 && split.rows < g.I) {
+        for (int64_t i0 = 0; i0 < g.I; i0 += split.rows) DLLM_TRY(launch_gemm(gemm_split_block(g, split.rows, i0), stream));
         return kOk;
     }
     if (vec && (ak != kADouble || ((g.lda % 2 == 0) && (reinterpret_cast<uintptr_t>(g.A) % 16 == 0)))) {

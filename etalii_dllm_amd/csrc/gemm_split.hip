@@ -1117,14 +1117,18 @@ bool split_parallel(const GemmCall& g) {
 // TFLOP/s) and 10 us of epilogue per window. FP64's round of 512 tiles of 128 x 128 takes 0.247 us per l, a last round of
 // at most one tile per CU 0.55 of that; launches of fewer tiles run at about 55 TFLOP/s. At 1023 x 8960 x 1536 the two
 // measure 370 and 600 us, at 2048 x 896 x 4864 285 and 310, at 1024 x 576 x 49152 (144 workgroups) 1.8 and 1.2 ms.
-bool split_pays(const GemmCall& g) {
+// In blocks of `rows` rows B is split once, and every block has its own passes and rounds.
+bool split_pays(const GemmCall& g, int64_t rows) {
     const double I = static_cast<double>(g.I), J = static_cast<double>(g.J), L = static_cast<double>(g.l1);
     const int64_t z = split_parallel(g) ? g.nseg : 1;
     const int64_t windows = g.seg ? g.nseg / z : 1;
-    const double r = static_cast<double>(ceil_div(g.I, kTile) * ceil_div(g.J, kTile) * z) / 512.0;
-    const double split = 50e-6 + (I + J) * L * 4e-12 +
-                         (r <= 1.0 ? 1.0 : r + 0.25) *
-                             (L / static_cast<double>(z) / 32.0 * 1.14e-6 + static_cast<double>(windows) * 10e-6);
+    const auto block = [&](int64_t n) {
+        const double r = static_cast<double>(ceil_div(n, kTile) * ceil_div(g.J, kTile) * z) / 512.0;
+        return 50e-6 + (r <= 1.0 ? 1.0 : r + 0.25) *
+                           (L / static_cast<double>(z) / 32.0 * 1.14e-6 + static_cast<double>(windows) * 10e-6);
+    };
+    const int64_t rest = g.I % rows;
+    const double split = (I + J) * L * 4e-12 + static_cast<double>(g.I / rows) * block(rows) + (rest ? block(rest) : 0.0);
     const int64_t big = ceil_div(g.I, 128) * ceil_div(g.J, 128) * z;
     const int64_t last = big % 512;
     const double fp64 = big >= 512 ? (static_cast<double>(big / 512) + (last == 0 ? 0.0 : last <= 256 ? 0.55 : 1.0)) *
@@ -1133,34 +1137,39 @@ bool split_pays(const GemmCall& g) {
     return split < 0.95 * fp64;
 }
 
-bool split_fits(const GemmCall& g) {
+// Whether the path takes the call's operands and reduction at all.
+bool split_takes(const GemmCall& g) {
     if (g.a_kind == 0 || g.l0 != 0 || g.l1 < 256 || g.I <= 0 || g.J <= 0) return false;
     if (g.seg == nullptr ? g.l1 > kMaxWindow && (g.a_kind != 2 || g.Bt == nullptr || g.bt_transpose != nullptr || g.l1 >= (1 << 30)) : g.seg_max <= 0 || g.seg_max > kMaxWindow || g.nseg > 64) return false;
-    if (g.l1 / kPartL + (g.seg ? g.nseg : 1) > 65535) return false;
-    return split_pays(g);
+    return g.l1 / kPartL + (g.seg ? g.nseg : 1) <= 65535;
 }
 
 }  // namespace
 
 size_t split_gemm_bytes(const GemmCall& g) {
-    return split_fits(g) ? split_layout(g, split_parallel(g) ? g.nseg : 1).bytes : 0;
+    return split_takes(g) && split_pays(g, g.I) ? split_layout(g, split_parallel(g) ? g.nseg : 1).bytes : 0;
 }
 
 SplitPlan split_plan(const GemmCall& g) {
     SplitPlan plan;
-    if (g.split_scratch == nullptr || !split_fits(g)) return plan;
+    if (g.split_scratch == nullptr || !split_takes(g)) return plan;
+    if (g.split_block) {  // decided with the whole call
+        plan.rows = g.I;
+        return plan;
+    }
+    if (!split_pays(g, g.I)) return plan;
     plan.parallel = split_parallel(g);
     if (split_layout(g, plan.parallel ? g.nseg : 1).bytes <= g.split_cap) {
         plan.rows = g.I;
         return plan;
     }
     if (plan.parallel) return plan;
-    // row blocks that share B
+    // the largest halving of the rows whose block fits: all blocks run here, or none
     GemmCall b = g;
     b.split_share = 2;
     for (b.I = (g.I / 2 + 127) / 128 * 128; b.I >= 1024; b.I = (b.I / 2 + 127) / 128 * 128)
         if (split_layout(b, 1).bytes <= g.split_cap) {
-            plan.rows = b.I;
+            if (split_pays(g, b.I)) plan.rows = b.I;
             return plan;
         }
     return plan;

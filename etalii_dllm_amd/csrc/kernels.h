@@ -60,11 +60,15 @@ struct GemmCall {
     // the call before, of the same share, reduction and windows, left it in the scratch.
     int split_share = 0;
     bool split_ready = false;
+    bool split_block = false;  // a row block of a call (gemm_split_block): on the int8 path, as decided for the call
     uint32_t* split_stat = nullptr;  // optional device counter: the tiles that the path hands back to FP64 are added
     int split_site = -1;             // the caller's own number of the call
 };
 // The rows of a block of the call on the int8 path: I when it runs there whole, 0 when it does not run there.
 int64_t gemm_split_rows(const GemmCall& g);
+// The block of at most `rows` (gemm_split_rows) rows from row i0. Every block runs on the int8 path, whatever its own
+// size, so each after the first finds B's split in the scratch.
+GemmCall gemm_split_block(const GemmCall& g, int64_t rows, int64_t i0);
 // Scratch bytes of the int8 path for the whole call (0: the shape does not take it).
 size_t split_gemm_bytes(const GemmCall& g);
 // Whether a float-A call runs on the matrix-core kernel (every operand row a whole number of 16-byte chunks).

@@ -23,3 +23,7 @@ def pytest_configure(config):
     oracle_so = ROOT / "oracle" / "liboracle.so"
     if not oracle_so.exists():
         subprocess.run(["make", "-C", str(ROOT / "oracle"), "liboracle.so"], check=True, capture_output=True)
+    from etalii_dllm_amd import build
+
+    if build.LIBRARY.exists() and not (ROOT / "tests" / "native" / "libmatmul_calls.so").exists():
+        build.build_test_calls()

@@ -1,0 +1,57 @@
+"""How a large matmul is split over the int8 path's scratch (csrc/gemm.hip, gemm_split.hip): host decisions, no GPU.
+
+A call that does not fit the scratch runs in row blocks that share B's split, which the first block makes. So either all
+of a call's blocks run on the int8 path or none, and only the first is without a split to take."""
+
+from __future__ import annotations
+
+import ctypes as C
+import random
+
+import pytest
+
+import matmul_calls as M
+
+pytestmark = pytest.mark.skipif(not M.HARNESS.exists(), reason="tests/native is not built")
+
+GIB = 1 << 30
+# calls whose full blocks, asked one by one, are quicker on FP64 while the smaller last block is not (its tiles fill the
+# last round of workgroups better): a head's input gradient, its forward and its windowed weight gradient, two layers'
+UNEVEN = [
+    M.row_major(33304, 256, 32000, cap=2 * GIB),
+    M.row_major(2308, 256000, 576, cap=GIB),
+    M.windowed(151936, 1536, 4600, 8, 575, cap=5 * GIB),
+    M.row_major(2912, 1452, 2888, cap=66501847),
+    M.windowed(2832, 1512, 5282, 6, 3169, cap=241863356),
+]
+
+
+def assert_blocks(h, call: M.MatmulCall):
+    made = M.blocks(h, call)
+    rows = h.matmul_rows(C.byref(call))
+    what = (call.I, call.J, call.L, call.nseg, call.cap, made)
+    if not rows:
+        return made
+    assert sum(b[0] for b in made) == call.I and all(b[0] == rows for b in made[:-1]), what
+    assert all(on_int8 == n for n, on_int8, _ in made), what
+    assert [ready for _, _, ready in made] == [0] + [1] * (len(made) - 1), what
+    return made
+
+
+@pytest.mark.parametrize("call", UNEVEN, ids=lambda c: f"{c.I}x{c.J}x{c.L}")
+def test_blocks_whose_last_alone_would_pay(call):
+    h = M.load()
+    made = assert_blocks(h, call)
+    assert len(made) > 1 and made[-1][0] < made[0][0]
+
+
+def test_blocks_of_any_call_and_scratch():
+    h, rng, several = M.load(), random.Random(7), 0
+    for _ in range(20000):
+        rows, cols, length = (int(2 ** rng.uniform(8, 17)) // 4 * 4 for _ in range(3))
+        nseg = rng.choice([0, 1, 2, 8, 64])
+        call = M.row_major(rows, cols, length) if rng.random() < 0.5 else \
+            M.windowed(rows, cols, length, nseg, min(length, 2 * length // max(nseg, 1)))
+        call.cap = int(h.matmul_bytes(C.byref(call)) * rng.uniform(0.05, 1.1))
+        several += len(assert_blocks(h, call)) > 1
+    assert several > 1000  # the sweep reaches what it is about
