@@ -956,14 +956,14 @@ struct dllm_hip_trainer {
 
     int c_head() const { return c.tie_embeddings ? emb : lm_head; }
 
-    // The call with the int8 path's scratch of its stream.
-    GemmCall with_split(const GemmCall& g, hipStream_t s) const {
+    // The call with the int8 path's scratch of its stream; rested: also where its matmul rests now.
+    GemmCall with_split(const GemmCall& g, hipStream_t s, bool rested = false) const {
         GemmCall c = g;
         // The layers' weight gradients stay on FP64: eight windows' epilogues, two column-ordered operands to split and copy,
         // and long-tailed gradients to recompute take 4.3 ms where FP64 takes 3.4 (8960 x 1536 over 8 x 1024).
         if (g.a_kind == 1 && g.C != G(c_head())) return c;
         if (split_stat != nullptr && g.split_site >= 0) {
-            if (split_rest[static_cast<size_t>(g.split_site)] > 0) return c;
+            if (!rested && split_rest[static_cast<size_t>(g.split_site)] > 0) return c;
             c.split_stat = split_stat + g.split_site;
         }
         const int k = side_on && s == side ? 1 : 0;
@@ -1080,13 +1080,25 @@ struct dllm_hip_trainer {
     static constexpr int kGroupCap = 3;  // matmuls per group table
     char* grp_tables = nullptr;          // [layer][kind]
     std::vector<GemmGroup> grp;          // [layer * kLayerGroups + kind]
-    bool grp_on[kLayerGroups] = {};
+    // [layer * kLayerGroups + kind]: the group can run (shapes, sizes), and which matmul's int8 path takes its place
+    // (split_site, or -1): the group then runs only while that matmul rests
+    struct GroupUse {
+        bool fits = false;
+        int int8_site = -1;
+    };
+    std::vector<GroupUse> grp_use;
     std::vector<double> grp_flops;       // algorithmic flop of each group (matmul timing)
     int64_t grp_rows = -1;               // the row count the tables were prepared for
     float *dh_b = nullptr, *dh_c = nullptr;
     float* dh1 = nullptr;  // the attention block's input gradient (dh holds the MLP block's)
 
     const GemmGroup& group_of(int64_t l, int kind) const { return grp[static_cast<size_t>(l * kLayerGroups + kind)]; }
+    // Whether layer l's matmuls of this kind run as one grouped launch in this step.
+    bool grouped(int64_t l, int kind, int64_t R) const {
+        if (grp_rows != R) return false;
+        const GroupUse& u = grp_use[static_cast<size_t>(l * kLayerGroups + kind)];
+        return u.fits && (u.int8_site < 0 || split_rest[static_cast<size_t>(u.int8_site)] > 0);
+    }
     const char* table_of(int64_t l, int kind) const {
         return grp_tables + gemm_group_bytes(kGroupCap) * static_cast<size_t>(l * kLayerGroups + kind);
     }
@@ -1099,16 +1111,16 @@ struct dllm_hip_trainer {
         std::vector<char> host(gb * n, 0);
         grp.assign(n, GemmGroup{});
         grp_flops.assign(n, 0.0);
+        grp_use.assign(n, GroupUse{});
         // the grouped kernel takes whole 16-byte chunks of the operands; other shapes keep one launch per matmul
         const bool rows_ok = R > 0 && H % 4 == 0;
-        for (int k = 0; k < kLayerGroups; ++k) grp_on[k] = rows_ok && (E == 0 || k == kGrpQkvFwd || k == kGrpQkvDx);
         const float* dqf = c.qk_norm ? dq2 : dq;
         const float* dkf = c.qk_norm ? dk2 : dk;
         for (int64_t l = 0; l < c.layers; ++l) {
             const LayerIds& L = layer_ids[static_cast<size_t>(l)];
             Saved& sv = saved[static_cast<size_t>(l)];
             for (int k = 0; k < kLayerGroups; ++k) {
-                if (!grp_on[k]) continue;
+                if (!rows_ok || (E > 0 && k != kGrpQkvFwd && k != kGrpQkvDx)) continue;
                 GemmCall calls[kGroupCap];
                 int nc = 0;
                 if (k == kGrpQkvFwd) {
@@ -1133,10 +1145,11 @@ struct dllm_hip_trainer {
                 const size_t gi = static_cast<size_t>(l * kLayerGroups + k);
                 if (ok) DLLM_TRY(gemm_group_prepare(calls, nc, kGroupCap, host.data() + gb * gi, &g));
                 for (int i = 0; i < nc; ++i) grp_flops[gi] += flops_of(calls[i]);
-                // the input-gradient groups only where the separate launches would take small tiles; none whose first
+                // the input-gradient groups only where the separate launches would take small tiles; not while the first
                 // matmul runs on the int8 path (the others then share its split of the rows)
                 const bool dx_kind = k == kGrpMlpDx || k == kGrpQkvDx;
-                if (!ok || (dx_kind && g.tile == 4) || gemm_split_rows(with_split(calls[0], s)) > 0) grp_on[k] = false;
+                grp_use[gi].fits = ok && !(dx_kind && g.tile == 4);
+                if (gemm_split_rows(with_split(calls[0], s, true)) > 0) grp_use[gi].int8_site = calls[0].split_site;
             }
         }
         DLLM_TRY(check_hip(hipStreamSynchronize(s), "group tables"));  // no launch still reads the old tables
@@ -1153,7 +1166,7 @@ struct dllm_hip_trainer {
     int qkv_forward(int64_t l, int64_t R, hipStream_t s) {
         const LayerIds& L = layer_ids[static_cast<size_t>(l)];
         Saved& sv = saved[static_cast<size_t>(l)];
-        if (grp_on[kGrpQkvFwd] && grp_rows == R) return group_launch(l, kGrpQkvFwd, s);
+        if (grouped(l, kGrpQkvFwd, R)) return group_launch(l, kGrpQkvFwd, s);
         const GemmCall calls[3] = {fwd_call(sv.h1, R, H, L.q, Popt(L.qb), sv.q_raw, nullptr),
                                    fwd_call(sv.h1, R, H, L.k, Popt(L.kb), sv.k_raw, nullptr),
                                    fwd_call(sv.h1, R, H, L.v, Popt(L.vb), sv.v, nullptr)};
@@ -1449,7 +1462,7 @@ struct dllm_hip_trainer {
         }
         if (pre_norms()) DLLM_TRY(launch_rms_norm(sv.x_mid, P(L.mlp_norm), sv.h2, R, H, eps, uo(), nullptr, s));
         if (sparse(l)) return moe_forward(l, R, x_out, s);
-        if (grp_on[kGrpMlpFwd] && grp_rows == R) {
+        if (grouped(l, kGrpMlpFwd, R)) {
             DLLM_TRY(group_launch(l, kGrpMlpFwd, s));
         } else {
             const GemmCall calls[2] = {fwd_call(sv.h2, R, H, L.gate, nullptr, sv.gate, nullptr),
@@ -1501,7 +1514,7 @@ struct dllm_hip_trainer {
             }
             DLLM_TRY(side_mark(kSideMlp));
             DLLM_TRY(side_wait(kSideNormMlp, s));  // the previous layer's mlp norm dW reads dh
-            if (grp_on[kGrpMlpDx] && grp_rows == R) {
+            if (grouped(l, kGrpMlpDx, R)) {
                 DLLM_TRY(group_launch(l, kGrpMlpDx, s));
                 DLLM_TRY(launch_add(dh, dh_b, dh, R * H, s));  // dh2 = dx_gate + dx_up
             } else {
@@ -1579,7 +1592,7 @@ struct dllm_hip_trainer {
         }
         DLLM_TRY(side_mark(kSideQkv));
         DLLM_TRY(side_wait(kSideNormAttn, s));  // the previous layer's attention norm dW reads dh1
-        if (grp_on[kGrpQkvDx] && grp_rows == R) {
+        if (grouped(l, kGrpQkvDx, R)) {
             DLLM_TRY(group_launch(l, kGrpQkvDx, s));
             DLLM_TRY(launch_add3(dh1, dh_b, dh_c, dh1, R * H, s));  // (dh_q + dh_k) + dh_v
         } else {

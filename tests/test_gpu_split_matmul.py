@@ -90,3 +90,50 @@ def test_linear_of_few_rows(K, kind, rows, inf, outf):
     b = operand("gauss", 9, 1, outf)[0]
     assert_same(K.linear(x, w, b), O.oracle_kernels().linear(x, w, b), "linear")
     assert_same(K.linear(x, w), K.linear(np.repeat(x, 80, axis=0), w)[::80], "the same rows in a larger call")
+
+
+@pytest.mark.parametrize("other_rows", [False, True])
+def test_a_resting_matmul_runs_grouped_and_comes_back(other_rows):
+    """A layer's gate and up projections hand every tile back once (a channel of great size meets zero weights, so the
+    results lie far below the operands' digits), rest for 32 steps as one grouped FP64 launch, and return to the int8
+    path as two calls, whatever row counts the steps between had. Counted by the matmul launches of a step."""
+    import ctypes as C
+
+    from etalii_dllm_amd import kernels
+    from etalii_dllm_amd.trainer import Decoder, Trainer
+
+    lib = kernels.lib
+    t = Trainer(Decoder(256, 896, 4864, 1, 14, 2, 64, 1e-6, 1e4, True), 2048, 2, 1024)
+    rng = np.random.default_rng(3)
+    dims = {"token_embedding": (256, 896), "q": (896, 896), "k": (128, 896), "v": (128, 896), "o": (896, 896),
+            "gate": (4864, 896), "up": (4864, 896), "down": (896, 4864)}
+    weights = {n: np.ones(896, np.float32) if n.endswith("norm.weight") else
+               (0.02 * rng.standard_normal(dims[n.split(".")[-2]])).astype(np.float32) for n in t.names}
+    for name in ("gate", "up"):
+        weights[f"layers.0.mlp.{name}.weight"][:, 0] = 0.0
+    hot = {**weights, "layers.0.mlp_norm.weight": weights["layers.0.mlp_norm.weight"].copy()}
+    hot["layers.0.mlp_norm.weight"][0] = 1e9
+    windows = {n: [rng.integers(0, 256, k + 1).tolist() for k in (1024, n - 1024)] for n in (2048, 2044)}
+    step = 0
+
+    def launches(rows: int) -> int:
+        nonlocal step
+        step += 1
+        kernels.check(lib.dllm_hip_trainer_profile(t.handle, 1))
+        t.step(windows[rows], 0.0, step, weight_decay=0.0)
+        n, ms, flops = C.c_int64(), C.c_double(), C.c_double()
+        kernels.check(lib.dllm_hip_trainer_profile_read(t.handle, C.byref(n), C.byref(ms), C.byref(flops)))
+        return n.value
+
+    lib.dllm_hip_trainer_profile.argtypes = [C.c_void_p, C.c_int]
+    lib.dllm_hip_trainer_profile_read.argtypes = [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_double),
+                                                  C.POINTER(C.c_double)]
+    t.load(weights)
+    apart = launches(2048)
+    t.load(hot)
+    assert launches(2048) == apart  # hands its tiles back
+    t.load(weights)
+    rows = 2044 if other_rows else 2048
+    assert [launches(rows) for _ in range(32)] == [apart - 1] * 32  # gate and up in one launch
+    assert [launches(rows) for _ in range(3)] == [apart] * 3
+    t.close()
