@@ -104,7 +104,7 @@ struct SplitParams {
     uint64_t* slots;
     float* slot_values;  // [slot][1 + nseg]
     uint32_t slot_cap;
-    uint32_t* stat;  // flagged tiles of the caller's (null: none kept)
+    uint32_t* stat;  // the caller's counts: flagged tiles, chains computed (null: none kept)
 };
 
 struct Window {
@@ -972,6 +972,7 @@ __global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2))) void s
     const bool owner = tid >= 256 && tid - 256 < kFixRows;  // the lanes that add
     const int row = owner ? tid - 256 : 0;
     const bool sequence = kSeg && !p.partial;
+    if (p.stat && blockIdx.x == 0 && tid == 0) atomicAdd(p.stat + 1, n);
     for (uint32_t k0 = blockIdx.x * kFixRows; k0 < n; k0 += gridDim.x * kFixRows) {
         const uint32_t k = k0 + static_cast<uint32_t>(row);
         const uint64_t item = k < n ? p.list[k] : ~uint64_t{0};
@@ -1118,7 +1119,7 @@ bool split_parallel(const GemmCall& g) {
 // at most one tile per CU 0.55 of that; launches of fewer tiles run at about 55 TFLOP/s. At 1023 x 8960 x 1536 the two
 // measure 370 and 600 us, at 2048 x 896 x 4864 285 and 310, at 1024 x 576 x 49152 (144 workgroups) 1.8 and 1.2 ms.
 // In blocks of `rows` rows B is split once, and every block has its own passes and rounds.
-bool split_pays(const GemmCall& g, int64_t rows) {
+SplitCost split_cost(const GemmCall& g, int64_t rows) {
     const double I = static_cast<double>(g.I), J = static_cast<double>(g.J), L = static_cast<double>(g.l1);
     const int64_t z = split_parallel(g) ? g.nseg : 1;
     const int64_t windows = g.seg ? g.nseg / z : 1;
@@ -1134,7 +1135,12 @@ bool split_pays(const GemmCall& g, int64_t rows) {
     const double fp64 = big >= 512 ? (static_cast<double>(big / 512) + (last == 0 ? 0.0 : last <= 256 ? 0.55 : 1.0)) *
                                          (L / static_cast<double>(z)) * 0.247e-6
                                    : 2.0 * I * J * L / 55e12;
-    return split < 0.95 * fp64;
+    return {fp64, split};
+}
+
+bool split_pays(const GemmCall& g, int64_t rows) {
+    const SplitCost c = split_cost(g, rows);
+    return c.split < 0.95 * c.fp64;
 }
 
 // Whether the path takes the call's operands and reduction at all.
@@ -1148,6 +1154,18 @@ bool split_takes(const GemmCall& g) {
 
 size_t split_gemm_bytes(const GemmCall& g) {
     return split_takes(g) && split_pays(g, g.I) ? split_layout(g, split_parallel(g) ? g.nseg : 1).bytes : 0;
+}
+
+SplitCost gemm_split_cost(const GemmCall& g) { return split_cost(g, gemm_split_rows(g)); }
+
+// A round of the 512 workgroups that recompute 32 chains each takes 9.6 ns per l (1030 x 1792 x 4320: 83 us for two, 1792 x
+// 1504 x 4320: 124 us for three). Handed-back tiles take at least one tile's reduction in FP64, 70 ns per l: under 160 of
+// 476 tiles of 1030 x 1792 x 36000 took 2.53 ms, as long as all of them in FP64 (2.61 ms).
+double gemm_split_redo_seconds(int64_t chain_l, int64_t tile_l, int64_t chains, int64_t tiles) {
+    const int64_t rounds = ceil_div(chains, 512 * kFixRows);  // the first is in split_cost's estimate
+    const double fix = static_cast<double>(rounds > 1 ? rounds - 1 : 0) * static_cast<double>(chain_l) * 9.6e-9;
+    const double redo = tiles == 0 ? 0.0 : static_cast<double>(tile_l) * std::max(70e-9, static_cast<double>(tiles) * 0.18e-9);
+    return fix + redo;
 }
 
 SplitPlan split_plan(const GemmCall& g) {

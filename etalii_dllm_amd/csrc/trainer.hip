@@ -211,14 +211,19 @@ struct dllm_hip_trainer {
     int64_t gemm_part_cap = 0;  // floats: per-window partials of the layer weight gradients
     char* split_mem[2] = {nullptr, nullptr};  // the int8 matmuls' scratch: the step's stream, the side stream
     size_t split_cap[2] = {0, 0};
-    // How the int8 path fares at each matmul of the step (3 x weight + forward, input gradient, weight gradient): the tiles
-    // it handed back in the step (device) of those it ran, and for how many steps more the matmul runs in FP64. Operands
-    // of very wide range (gradients of a batch learnt by heart) hand most tiles back, at the cost of both paths.
+    // How the int8 path fares at each matmul of the step (3 x weight + forward, input gradient, weight gradient). What it
+    // recomputes depends on the operands: long-tailed ones (an MLP's products, gradients of a batch learnt by heart) leave
+    // many outputs to their chains and hand tiles back to FP64, which can cost more than the path saves. The device counts
+    // both; a matmul whose recomputation took longer than its expected gain runs in FP64 for the next kSplitRest steps.
     static constexpr int kSplitRest = 32;
-    uint32_t* split_stat = nullptr;
-    std::vector<uint32_t> split_handed;
-    std::vector<int64_t> split_tiles;
-    std::vector<int> split_rest;
+    struct SplitSite {
+        SplitCost cost;                    // expected, of the step's calls so far
+        int64_t chain_l = 0, tile_l = 0;   // the lengths of an output's chain and of a tile's reduction
+        int rest = 0;                      // steps left in FP64
+    };
+    uint32_t* split_stat = nullptr;  // [site][2]: tiles handed back, chains computed
+    std::vector<uint32_t> split_done;
+    std::vector<SplitSite> split_sites;
     std::unordered_map<int64_t, int> tensor_at;  // by offset in the arenas
     // routed experts: E experts, K per token, EI expert intermediate size; shared buffers of the grouped rows
     int64_t E = 0, K = 0, EI = 0, RK = 0;
@@ -945,11 +950,10 @@ struct dllm_hip_trainer {
         if (split_cap[0] > 0) DLLM_TRY(make(&split_mem[0], split_cap[0]));
         if (split_cap[0] == 0) return kOk;
         const size_t sites = 3 * tensors.size();
-        DLLM_TRY(make(&split_stat, sites));
-        DLLM_TRY(check_hip(hipMemset(split_stat, 0, sites * sizeof(uint32_t)), "memset"));
-        split_handed.assign(sites, 0);
-        split_tiles.assign(sites, 0);
-        split_rest.assign(sites, 0);
+        DLLM_TRY(make(&split_stat, 2 * sites));
+        DLLM_TRY(check_hip(hipMemset(split_stat, 0, 2 * sites * sizeof(uint32_t)), "memset"));
+        split_done.assign(2 * sites, 0);
+        split_sites.assign(sites, SplitSite{});
         for (size_t i = 0; i < tensors.size(); ++i) tensor_at[tensors[i].offset] = static_cast<int>(i);
         return kOk;
     }
@@ -963,8 +967,8 @@ struct dllm_hip_trainer {
         // and long-tailed gradients to recompute take 4.3 ms where FP64 takes 3.4 (8960 x 1536 over 8 x 1024).
         if (g.a_kind == 1 && g.C != G(c_head())) return c;
         if (split_stat != nullptr && g.split_site >= 0) {
-            if (!rested && split_rest[static_cast<size_t>(g.split_site)] > 0) return c;
-            c.split_stat = split_stat + g.split_site;
+            if (!rested && split_sites[static_cast<size_t>(g.split_site)].rest > 0) return c;
+            c.split_stat = split_stat + 2 * g.split_site;
         }
         const int k = side_on && s == side ? 1 : 0;
         c.split_scratch = split_mem[k];
@@ -972,21 +976,29 @@ struct dllm_hip_trainer {
         return c;
     }
 
-    // After a step's synchronisation: matmuls that handed back more than a third of their tiles rest.
+    // After a step's synchronisation: matmuls whose recomputation cost more than the path gained rest. A gain below an eighth
+    // of the FP64 time is within what the two estimates are off by and counts as that eighth.
     int split_review(hipStream_t s) {
         if (split_stat == nullptr) return kOk;
-        for (size_t i = 0; i < split_handed.size(); ++i) {
-            if (split_rest[i] > 0) --split_rest[i];
-            if (3 * static_cast<int64_t>(split_handed[i]) > split_tiles[i]) split_rest[i] = kSplitRest;
-            split_tiles[i] = 0;
+        for (size_t i = 0; i < split_sites.size(); ++i) {
+            SplitSite& site = split_sites[i];
+            if (site.rest > 0) --site.rest;
+            const double gain = std::max(site.cost.fp64 - site.cost.split, site.cost.fp64 / 8.0);
+            if (gemm_split_redo_seconds(site.chain_l, site.tile_l, split_done[2 * i + 1], split_done[2 * i]) > gain)
+                site.rest = kSplitRest;
+            site.cost = SplitCost{};
         }
-        return check_hip(hipMemsetAsync(split_stat, 0, split_handed.size() * sizeof(uint32_t), s), "memset");
+        return check_hip(hipMemsetAsync(split_stat, 0, split_done.size() * sizeof(uint32_t), s), "memset");
     }
 
     int gemm(const GemmCall& g, hipStream_t s) {
         if (split_stat != nullptr && g.split_site >= 0 && gemm_split_rows(with_split(g, s)) > 0) {
-            const int64_t tiles = ceil_div(g.I, 64) * ceil_div(g.J, 64);  // of each window, where they run in parallel
-            split_tiles[static_cast<size_t>(g.split_site)] += tiles * (g.seg && tiles < 2048 ? g.nseg : 1);
+            SplitSite& site = split_sites[static_cast<size_t>(g.split_site)];
+            const SplitCost cost = gemm_split_cost(with_split(g, s));
+            site.cost.fp64 += cost.fp64;
+            site.cost.split += cost.split;
+            site.chain_l = g.seg ? g.l1 / g.nseg : g.l1;
+            site.tile_l = g.l1;
         }
         if (!profiling) return launch_gemm(with_split(g, s), s);
         DLLM_TRY(profile_begin(s));
@@ -1097,7 +1109,7 @@ struct dllm_hip_trainer {
     bool grouped(int64_t l, int kind, int64_t R) const {
         if (grp_rows != R) return false;
         const GroupUse& u = grp_use[static_cast<size_t>(l * kLayerGroups + kind)];
-        return u.fits && (u.int8_site < 0 || split_rest[static_cast<size_t>(u.int8_site)] > 0);
+        return u.fits && (u.int8_site < 0 || split_sites[static_cast<size_t>(u.int8_site)].rest > 0);
     }
     const char* table_of(int64_t l, int kind) const {
         return grp_tables + gemm_group_bytes(kGroupCap) * static_cast<size_t>(l * kLayerGroups + kind);
@@ -2105,7 +2117,7 @@ struct dllm_hip_trainer {
             DLLM_TRY(check_hip(hipMemcpyAsync(&route_flag, route_err, sizeof route_flag, hipMemcpyDeviceToHost, s),
                                "download"));
         if (split_stat != nullptr)
-            DLLM_TRY(check_hip(hipMemcpyAsync(split_handed.data(), split_stat, split_handed.size() * sizeof(uint32_t),
+            DLLM_TRY(check_hip(hipMemcpyAsync(split_done.data(), split_stat, split_done.size() * sizeof(uint32_t),
                                               hipMemcpyDeviceToHost, s), "download"));
         DLLM_TRY(check_hip(hipStreamSynchronize(s), "step"));
         DLLM_TRY(split_review(s));

@@ -92,11 +92,12 @@ def test_linear_of_few_rows(K, kind, rows, inf, outf):
     assert_same(K.linear(x, w), K.linear(np.repeat(x, 80, axis=0), w)[::80], "the same rows in a larger call")
 
 
-@pytest.mark.parametrize("other_rows", [False, True])
-def test_a_resting_matmul_runs_grouped_and_comes_back(other_rows):
-    """A layer's gate and up projections hand every tile back once (a channel of great size meets zero weights, so the
-    results lie far below the operands' digits), rest for 32 steps as one grouped FP64 launch, and return to the int8
-    path as two calls, whatever row counts the steps between had. Counted by the matmul launches of a step."""
+@pytest.mark.parametrize("other_rows,hot_rows", [(False, 2048), (True, 2048), (False, 512)])
+def test_a_resting_matmul_runs_grouped_and_comes_back(other_rows, hot_rows):
+    """A layer's gate and up projections hand the tiles of hot_rows rows back once (a channel of great size meets zero
+    weights, so the results lie far below the operands' digits), which costs more than the path saves. They rest for 32
+    steps as one grouped FP64 launch, and return to the int8 path as two calls, whatever row counts the steps between had.
+    Counted by the matmul launches of a step."""
     import ctypes as C
 
     from etalii_dllm_amd import kernels
@@ -111,9 +112,12 @@ def test_a_resting_matmul_runs_grouped_and_comes_back(other_rows):
                (0.02 * rng.standard_normal(dims[n.split(".")[-2]])).astype(np.float32) for n in t.names}
     for name in ("gate", "up"):
         weights[f"layers.0.mlp.{name}.weight"][:, 0] = 0.0
+    weights["layers.0.attention.o.weight"][0] = 0.0  # the channel is the embedding's: tokens of 128 and above have none
+    weights["token_embedding.weight"][128:, 0] = 0.0
     hot = {**weights, "layers.0.mlp_norm.weight": weights["layers.0.mlp_norm.weight"].copy()}
     hot["layers.0.mlp_norm.weight"][0] = 1e9
-    windows = {n: [rng.integers(0, 256, k + 1).tolist() for k in (1024, n - 1024)] for n in (2048, 2044)}
+    tokens = np.concatenate([rng.integers(0, 128, hot_rows), rng.integers(128, 256, 2049 - hot_rows)]).tolist()
+    windows = {n: [tokens[:1025], tokens[1024:n + 1]] for n in (2048, 2044)}
     step = 0
 
     def launches(rows: int) -> int:
