@@ -1158,11 +1158,11 @@ size_t split_gemm_bytes(const GemmCall& g) {
 
 SplitCost gemm_split_cost(const GemmCall& g) { return split_cost(g, gemm_split_rows(g)); }
 
-// A round of the 512 workgroups that recompute 32 chains each takes 9.6 ns per l (1030 x 1792 x 4320: 83 us for two, 1792 x
+// Every 256 workgroups' worth of 32 chains take 9.6 ns per l (1030 x 1792 x 4320: 83 us for two rounds, 1792 x
 // 1504 x 4320: 124 us for three). Handed-back tiles take at least one tile's reduction in FP64, 70 ns per l: under 160 of
 // 476 tiles of 1030 x 1792 x 36000 took 2.53 ms, as long as all of them in FP64 (2.61 ms).
 double gemm_split_redo_seconds(int64_t chain_l, int64_t tile_l, int64_t chains, int64_t tiles) {
-    const int64_t rounds = ceil_div(chains, 512 * kFixRows);  // the first is in split_cost's estimate
+    const int64_t rounds = ceil_div(chains, 256 * kFixRows);  // the first is in split_cost's estimate
     const double fix = static_cast<double>(rounds > 1 ? rounds - 1 : 0) * static_cast<double>(chain_l) * 9.6e-9;
     const double redo = tiles == 0 ? 0.0 : static_cast<double>(tile_l) * std::max(70e-9, static_cast<double>(tiles) * 0.18e-9);
     return fix + redo;
