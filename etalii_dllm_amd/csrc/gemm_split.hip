@@ -104,7 +104,7 @@ struct SplitParams {
     uint64_t* slots;
     float* slot_values;  // [slot][1 + nseg]
     uint32_t slot_cap;
-    uint32_t* stat;  // the caller's counts: flagged tiles, chains computed (null: none kept)
+    uint32_t* stat;  // the caller's SplitDone (null: none kept)
 };
 
 struct Window {
@@ -1135,7 +1135,8 @@ SplitCost split_cost(const GemmCall& g, int64_t rows) {
     const double fp64 = big >= 512 ? (static_cast<double>(big / 512) + (last == 0 ? 0.0 : last <= 256 ? 0.55 : 1.0)) *
                                          (L / static_cast<double>(z)) * 0.247e-6
                                    : 2.0 * I * J * L / 55e12;
-    return {fp64, split};
+    return {fp64, split, g.seg ? L / static_cast<double>(g.nseg) : L, L * static_cast<double>(ceil_div(g.I, rows)),
+            g.seg != nullptr && z == 1};
 }
 
 bool split_pays(const GemmCall& g, int64_t rows) {
@@ -1158,14 +1159,19 @@ size_t split_gemm_bytes(const GemmCall& g) {
 
 SplitCost gemm_split_cost(const GemmCall& g) { return split_cost(g, gemm_split_rows(g)); }
 
-// Every 256 workgroups' worth of 32 chains take 9.6 ns per l (1030 x 1792 x 4320: 83 us for two rounds, 1792 x
-// 1504 x 4320: 124 us for three). Handed-back tiles take at least one tile's reduction in FP64, 70 ns per l: under 160 of
-// 476 tiles of 1030 x 1792 x 36000 took 2.53 ms, as long as all of them in FP64 (2.61 ms).
-double gemm_split_redo_seconds(int64_t chain_l, int64_t tile_l, int64_t chains, int64_t tiles) {
-    const int64_t rounds = ceil_div(chains, 256 * kFixRows);  // the first is in split_cost's estimate
-    const double fix = static_cast<double>(rounds > 1 ? rounds - 1 : 0) * static_cast<double>(chain_l) * 9.6e-9;
-    const double redo = tiles == 0 ? 0.0 : static_cast<double>(tile_l) * std::max(70e-9, static_cast<double>(tiles) * 0.18e-9);
-    return fix + redo;
+// Every 256 workgroups' worth of 32 chains take 9.6 ns per l (1030 x 1792 x 4320: 83 us for two rounds, 1792 x 1504 x 4320: 124
+// us for three); the first round is in split_cost's estimate. Handed-back tiles, however few, take a tile's whole reduction
+// in FP64, 70 to 130 ns per l: fewer than 160 of 476 tiles of 1030 x 1792 x 36000 took 2.53 ms (all of them in FP64 2.61),
+// some of 4096 x 1536 x 151936 took 19.6 ms (29). In a sequence of windows an open output also costs its slot, 2 ns and
+// more: the logits' gradient of 8192 rows and 151936 words times hidden 1536, 8 windows, takes 47.8 ms with 0.7 million
+// chains (flat logits), 53.1 with 2.4 (logits of deviation 0.78), 73.6 with 3.4 (1.2), 113 with 4.4 (2), and 55.5 in FP64.
+// A gain below an eighth of the FP64 time is within what the two estimates are off by and counts as that eighth.
+bool gemm_split_lost(const SplitCost& c, const SplitDone& d) {
+    const int64_t rounds = ceil_div(static_cast<int64_t>(d.chains), 256 * kFixRows);
+    double t = static_cast<double>(rounds > 1 ? rounds - 1 : 0) * c.chain_l * 9.6e-9;
+    if (c.sequence) t += static_cast<double>(d.chains) * 2.5e-9;
+    if (d.tiles > 0) t += std::min(c.fp64, c.tile_l * std::max(130e-9, static_cast<double>(d.tiles) * 0.18e-9));
+    return t > std::max(c.fp64 - c.split, c.fp64 / 8.0);
 }
 
 SplitPlan split_plan(const GemmCall& g) {

@@ -61,8 +61,7 @@ struct GemmCall {
     int split_share = 0;
     bool split_ready = false;
     bool split_block = false;  // a row block of a call (gemm_split_block): on the int8 path, as decided for the call
-    // optional device counters, added to: the tiles that the path hands back to FP64, the outputs it recomputes by their chains
-    uint32_t* split_stat = nullptr;
+    uint32_t* split_stat = nullptr;  // optional SplitDone in device memory, which the call adds to
     int split_site = -1;             // the caller's own number of the call
 };
 // The rows of a block of the call on the int8 path: I when it runs there whole, 0 when it does not run there.
@@ -70,13 +69,19 @@ int64_t gemm_split_rows(const GemmCall& g);
 // The block of at most `rows` (gemm_split_rows) rows from row i0. Every block runs on the int8 path, whatever its own
 // size, so each after the first finds B's split in the scratch.
 GemmCall gemm_split_block(const GemmCall& g, int64_t rows, int64_t i0);
-// What the call, one that the int8 path takes, is expected to cost in FP64 and there (with few outputs to recompute), and
-// what it costs beyond that when `chains` outputs of chain_l products and `tiles` 64 x 64 tiles of tile_l are recomputed.
+// What the call, one that the int8 path takes, is expected to cost in FP64 and there, with few outputs to recompute ...
 struct SplitCost {
     double fp64 = 0.0, split = 0.0;  // seconds
+    double chain_l = 0.0, tile_l = 0.0;  // the mean length of an output's chain; a tile's reduction, in each row block
+    bool sequence = false;           // windows in sequence
 };
 SplitCost gemm_split_cost(const GemmCall& g);
-double gemm_split_redo_seconds(int64_t chain_l, int64_t tile_l, int64_t chains, int64_t tiles);
+// ... and the work that its operands then made.
+struct SplitDone {
+    uint32_t tiles = 0, chains = 0;  // handed back to FP64, outputs recomputed by their chains
+};
+// Whether that work took longer than the path was to save.
+bool gemm_split_lost(const SplitCost& cost, const SplitDone& done);
 // Scratch bytes of the int8 path for the whole call (0: the shape does not take it).
 size_t split_gemm_bytes(const GemmCall& g);
 // Whether a float-A call runs on the matrix-core kernel (every operand row a whole number of 16-byte chunks).

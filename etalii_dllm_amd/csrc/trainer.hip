@@ -217,12 +217,11 @@ struct dllm_hip_trainer {
     // both; a matmul whose recomputation took longer than its expected gain runs in FP64 for the next kSplitRest steps.
     static constexpr int kSplitRest = 32;
     struct SplitSite {
-        SplitCost cost;                    // expected, of the step's calls so far
-        int64_t chain_l = 0, tile_l = 0;   // the lengths of an output's chain and of a tile's reduction
-        int rest = 0;                      // steps left in FP64
+        SplitCost cost;  // expected, of the step's calls so far
+        int rest = 0;    // steps left in FP64
     };
-    uint32_t* split_stat = nullptr;  // [site][2]: tiles handed back, chains computed
-    std::vector<uint32_t> split_done;
+    SplitDone* split_stat = nullptr;  // per site (device)
+    std::vector<SplitDone> split_done;
     std::vector<SplitSite> split_sites;
     std::unordered_map<int64_t, int> tensor_at;  // by offset in the arenas
     // routed experts: E experts, K per token, EI expert intermediate size; shared buffers of the grouped rows
@@ -950,9 +949,9 @@ struct dllm_hip_trainer {
         if (split_cap[0] > 0) DLLM_TRY(make(&split_mem[0], split_cap[0]));
         if (split_cap[0] == 0) return kOk;
         const size_t sites = 3 * tensors.size();
-        DLLM_TRY(make(&split_stat, 2 * sites));
-        DLLM_TRY(check_hip(hipMemset(split_stat, 0, 2 * sites * sizeof(uint32_t)), "memset"));
-        split_done.assign(2 * sites, 0);
+        DLLM_TRY(make(&split_stat, sites));
+        DLLM_TRY(check_hip(hipMemset(split_stat, 0, sites * sizeof(SplitDone)), "memset"));
+        split_done.assign(sites, SplitDone{});
         split_sites.assign(sites, SplitSite{});
         for (size_t i = 0; i < tensors.size(); ++i) tensor_at[tensors[i].offset] = static_cast<int>(i);
         return kOk;
@@ -968,7 +967,7 @@ struct dllm_hip_trainer {
         if (g.a_kind == 1 && g.C != G(c_head())) return c;
         if (split_stat != nullptr && g.split_site >= 0) {
             if (!rested && split_sites[static_cast<size_t>(g.split_site)].rest > 0) return c;
-            c.split_stat = split_stat + 2 * g.split_site;
+            c.split_stat = reinterpret_cast<uint32_t*>(split_stat + g.split_site);
         }
         const int k = side_on && s == side ? 1 : 0;
         c.split_scratch = split_mem[k];
@@ -976,29 +975,25 @@ struct dllm_hip_trainer {
         return c;
     }
 
-    // After a step's synchronisation: matmuls whose recomputation cost more than the path gained rest. A gain below an eighth
-    // of the FP64 time is within what the two estimates are off by and counts as that eighth.
+    // After a step's synchronisation: matmuls whose recomputation cost more than the path gained rest.
     int split_review(hipStream_t s) {
         if (split_stat == nullptr) return kOk;
         for (size_t i = 0; i < split_sites.size(); ++i) {
             SplitSite& site = split_sites[i];
             if (site.rest > 0) --site.rest;
-            const double gain = std::max(site.cost.fp64 - site.cost.split, site.cost.fp64 / 8.0);
-            if (gemm_split_redo_seconds(site.chain_l, site.tile_l, split_done[2 * i + 1], split_done[2 * i]) > gain)
-                site.rest = kSplitRest;
+            if (gemm_split_lost(site.cost, split_done[i])) site.rest = kSplitRest;
             site.cost = SplitCost{};
         }
-        return check_hip(hipMemsetAsync(split_stat, 0, split_done.size() * sizeof(uint32_t), s), "memset");
+        return check_hip(hipMemsetAsync(split_stat, 0, split_done.size() * sizeof(SplitDone), s), "memset");
     }
 
     int gemm(const GemmCall& g, hipStream_t s) {
         if (split_stat != nullptr && g.split_site >= 0 && gemm_split_rows(with_split(g, s)) > 0) {
             SplitSite& site = split_sites[static_cast<size_t>(g.split_site)];
-            const SplitCost cost = gemm_split_cost(with_split(g, s));
-            site.cost.fp64 += cost.fp64;
-            site.cost.split += cost.split;
-            site.chain_l = g.seg ? g.l1 / g.nseg : g.l1;
-            site.tile_l = g.l1;
+            SplitCost cost = gemm_split_cost(with_split(g, s));
+            cost.fp64 += site.cost.fp64;
+            cost.split += site.cost.split;
+            site.cost = cost;
         }
         if (!profiling) return launch_gemm(with_split(g, s), s);
         DLLM_TRY(profile_begin(s));
@@ -2117,7 +2112,7 @@ struct dllm_hip_trainer {
             DLLM_TRY(check_hip(hipMemcpyAsync(&route_flag, route_err, sizeof route_flag, hipMemcpyDeviceToHost, s),
                                "download"));
         if (split_stat != nullptr)
-            DLLM_TRY(check_hip(hipMemcpyAsync(split_done.data(), split_stat, split_done.size() * sizeof(uint32_t),
+            DLLM_TRY(check_hip(hipMemcpyAsync(split_done.data(), split_stat, split_done.size() * sizeof(SplitDone),
                                               hipMemcpyDeviceToHost, s), "download"));
         DLLM_TRY(check_hip(hipStreamSynchronize(s), "step"));
         DLLM_TRY(split_review(s));

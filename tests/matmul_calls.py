@@ -24,6 +24,7 @@ def load(path: Path = HARNESS) -> C.CDLL:
     for name in ("matmul_rows", "matmul_bytes", "matmul_blocks"):
         getattr(h, name).restype = _N
     h.matmul_blocks.argtypes = [C.POINTER(MatmulCall), _N] + [C.POINTER(_N)] * 3
+    h.matmul_lost.argtypes = [C.POINTER(MatmulCall), C.c_uint32, C.c_uint32]
     h.matmul_run.argtypes = [C.POINTER(MatmulCall), _P]
     return h
 

@@ -85,6 +85,11 @@ int64_t matmul_blocks(const MatmulCall* m, int64_t most, int64_t* rows, int64_t*
     return k;
 }
 
+// Whether the call, having handed back `tiles` and recomputed `chains` outputs, lost time on the int8 path.
+int matmul_lost(const MatmulCall* m, uint32_t tiles, uint32_t chains) {
+    return gemm_split_lost(gemm_split_cost(call_of(*m)), SplitDone{tiles, chains});
+}
+
 int matmul_run(const MatmulCall* m, hipStream_t stream) { return launch_gemm(call_of(*m), stream); }
 
 }  // extern "C"

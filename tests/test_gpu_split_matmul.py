@@ -5,9 +5,12 @@ exact ties, zero rows, infinities and NaNs, so that every way an output is decid
 
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
+import matmul_calls as M
 import oracle_lib as O
 
 pytestmark = pytest.mark.gpu
@@ -98,16 +101,18 @@ def test_a_resting_matmul_runs_grouped_and_comes_back(other_rows, hot_rows):
     weights, so the results lie far below the operands' digits), which costs more than the path saves. They rest for 32
     steps as one grouped FP64 launch, and return to the int8 path as two calls, whatever row counts the steps between had.
     Counted by the matmul launches of a step."""
-    import ctypes as C
-
     from etalii_dllm_amd import kernels
     from etalii_dllm_amd.trainer import Decoder, Trainer
 
     lib = kernels.lib
-    t = Trainer(Decoder(256, 896, 4864, 1, 14, 2, 64, 1e-6, 1e4, True), 2048, 2, 1024)
+    h = M.load()
+    for n in (2048, 2044):  # of the layer's matmuls these two alone are the int8 path's
+        assert h.matmul_rows(C.byref(M.row_major(n, 3712, 896))) == n
+        assert not any(h.matmul_rows(C.byref(M.row_major(n, *s))) for s in ((896, 3712), (896, 896)))
+    t = Trainer(Decoder(256, 896, 3712, 1, 14, 2, 64, 1e-6, 1e4, True), 2048, 2, 1024)
     rng = np.random.default_rng(3)
     dims = {"token_embedding": (256, 896), "q": (896, 896), "k": (128, 896), "v": (128, 896), "o": (896, 896),
-            "gate": (4864, 896), "up": (4864, 896), "down": (896, 4864)}
+            "gate": (3712, 896), "up": (3712, 896), "down": (896, 3712)}
     weights = {n: np.ones(896, np.float32) if n.endswith("norm.weight") else
                (0.02 * rng.standard_normal(dims[n.split(".")[-2]])).astype(np.float32) for n in t.names}
     for name in ("gate", "up"):

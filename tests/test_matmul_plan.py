@@ -55,3 +55,27 @@ def test_blocks_of_any_call_and_scratch():
         call.cap = int(h.matmul_bytes(C.byref(call)) * rng.uniform(0.05, 1.1))
         several += len(assert_blocks(h, call)) > 1
     assert several > 1000  # the sweep reaches what it is about
+
+
+# measured: a call, the tiles it handed back and the outputs it recomputed, its milliseconds on the int8 path and on FP64
+MEASURED = [
+    (M.windowed(151936, 1536, 8192, 8, 1024, cap=5 * GIB), 0, 689183, 47.8, 55.5),  # the logits' gradient: flat logits ...
+    (M.windowed(151936, 1536, 8192, 8, 1024, cap=5 * GIB), 0, 2383861, 53.1, 55.4),
+    (M.windowed(151936, 1536, 8192, 8, 1024, cap=5 * GIB), 0, 3414249, 73.6, 55.5),
+    (M.windowed(151936, 1536, 8192, 8, 1024, cap=5 * GIB), 0, 4395842, 112.9, 55.4),  # ... to peaked ones
+    (M.windowed(50304, 2048, 8192, 4, 2048), 0, 243911, 18.0, 24.4),
+    (M.windowed(50304, 2048, 8192, 4, 2048), 0, 1967082, 48.3, 24.3),
+    (M.windowed(32768, 1536, 8192, 8, 1024), 0, 990948, 25.3, 11.9),
+    (M.windowed(65536, 1024, 2048, 2, 1024), 0, 343055, 6.2, 4.0),
+    (M.row_major(1918, 1056, 3232), 0, 12000, 0.265, 0.244),  # an MLP's product through its down projection
+    (M.row_major(8192, 1536, 8960), 0, 57000, 3.05, 3.77),
+    (M.row_major(8192, 1536, 151936, cap=5 * GIB), 100, 24000, 78.0, 58.0),  # a few handed-back tiles of a long reduction
+    (M.row_major(1030, 1792, 36000), 150, 16384, 4.2, 2.6),
+]
+
+
+@pytest.mark.parametrize("call,tiles,chains,int8,fp64", MEASURED, ids=lambda v: f"{v.I}x{v.J}x{v.L}" if hasattr(v, "I") else None)
+def test_recomputation_that_costs_more_than_the_path_saves(call, tiles, chains, int8, fp64):
+    h = M.load()
+    assert h.matmul_rows(C.byref(call)) > 0
+    assert bool(h.matmul_lost(C.byref(call), tiles, chains)) == (int8 > fp64)
