@@ -27,7 +27,6 @@
 #include <map>
 #include <memory>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
 #include "attn_step.h"
@@ -209,8 +208,8 @@ struct dllm_hip_trainer {
           *dgate = nullptr, *dup = nullptr, *col_part = nullptr, *col_part_side = nullptr, *emb_rows = nullptr,
           *gemm_part = nullptr;
     int64_t gemm_part_cap = 0;  // floats: per-window partials of the layer weight gradients
-    char* split_mem[2] = {nullptr, nullptr};  // the int8 matmuls' scratch: the step's stream, the side stream
-    size_t split_cap[2] = {0, 0};
+    char* split_mem = nullptr;  // the int8 matmuls' scratch, of the step's stream
+    size_t split_cap = 0;
     // How the int8 path fares at each matmul of the step (3 x weight + forward, input gradient, weight gradient). What it
     // recomputes depends on the operands: long-tailed ones (an MLP's products, gradients of a batch learnt by heart) leave
     // many outputs to their chains and hand tiles back to FP64, which can cost more than the path saves. The device counts
@@ -223,7 +222,6 @@ struct dllm_hip_trainer {
     SplitDone* split_stat = nullptr;  // per site (device)
     std::vector<SplitDone> split_done;
     std::vector<SplitSite> split_sites;
-    std::unordered_map<int64_t, int> tensor_at;  // by offset in the arenas
     // routed experts: E experts, K per token, EI expert intermediate size; shared buffers of the grouped rows
     int64_t E = 0, K = 0, EI = 0, RK = 0;
     float *xg = nullptr, *dyg = nullptr, *dxg = nullptr, *dweights = nullptr, *dlogits_r = nullptr, *dprob = nullptr,
@@ -909,17 +907,19 @@ struct dllm_hip_trainer {
         return kOk;
     }
 
-    // The most scratch an int8 matmul of a full step takes (side: of the layers' weight gradients), and the cap on it:
-    // a larger call runs in row blocks, at 8192 x 151936 logits two for the head's input gradient (768 tiles each) and
-    // three for its weight gradient.
+    // The cap on the int8 matmuls' scratch: a larger call runs in row blocks, at 8192 x 151936 logits and hidden 1536 two
+    // for the head's input gradient (1536 tiles of 64 x 64 each) and four for its weight gradient.
     static constexpr size_t kSplitMax = size_t{5} << 30;
 
-    size_t split_bytes(bool side_stream) const {
+    int head_id() const { return c.tie_embeddings ? emb : lm_head; }
+
+    // The most scratch that an int8 matmul of a full step takes: every forward matmul and input gradient, and the head's
+    // weight gradient (with_split).
+    size_t split_bytes() const {
         size_t most = 0;
-        const int head = c.tie_embeddings ? emb : lm_head;
         for (size_t i = 0; i < tensors.size(); ++i) {
             const TensorInfo& t = tensors[i];
-            if (t.wt_offset < 0 || (side_stream && static_cast<int>(i) == head)) continue;
+            if (t.wt_offset < 0) continue;
             GemmCall fwd, dx, dw;
             fwd.a_kind = dx.a_kind = 2;
             fwd.I = dx.I = dw.l1 = R_max;
@@ -932,46 +932,43 @@ struct dllm_hip_trainer {
             dw.seg_max = T_max;
             dw.seg_partial = gemm_part;
             dw.seg_partial_cap = gemm_part_cap;
-            if (!side_stream) most = std::max({most, split_gemm_bytes(fwd), split_gemm_bytes(dx)});
-            most = std::max(most, split_gemm_bytes(dw));
+            most = std::max({most, split_gemm_bytes(fwd), split_gemm_bytes(dx)});
+            if (static_cast<int>(i) == head_id()) most = std::max(most, split_gemm_bytes(dw));
         }
         return most;
     }
 
-    // The int8 path's scratch, after everything else: of the memory that is left at most half for each stream, 2 GiB kept
-    // free (a trainer that fits without it is made without it; its matmuls then run in smaller row blocks or in FP64).
+    // The int8 path's scratch, after everything else and of the memory that is left, 2 GiB kept free: a trainer that fits
+    // without it is made without it, and its matmuls then run in smaller row blocks or in FP64.
     int split_setup() {
         size_t free_bytes = 0, total_bytes = 0;
         DLLM_TRY(check_hip(hipMemGetInfo(&free_bytes, &total_bytes), "hipMemGetInfo"));
-        const size_t keep = size_t{2} << 30, left = free_bytes > keep ? (free_bytes - keep) / 2 : 0;
-        // the step's stream only: what runs on the side stream, the layers' weight gradients, stays on FP64
-        split_cap[0] = std::min({split_bytes(false), kSplitMax, left});
-        if (split_cap[0] > 0) DLLM_TRY(make(&split_mem[0], split_cap[0]));
-        if (split_cap[0] == 0) return kOk;
+        const size_t keep = size_t{2} << 30, left = free_bytes > keep ? free_bytes - keep : 0;
+        split_cap = std::min({split_bytes(), kSplitMax, left});
+        if (split_cap == 0) return kOk;
+        DLLM_TRY(make(&split_mem, split_cap));
         const size_t sites = 3 * tensors.size();
         DLLM_TRY(make(&split_stat, sites));
         DLLM_TRY(check_hip(hipMemset(split_stat, 0, sites * sizeof(SplitDone)), "memset"));
         split_done.assign(sites, SplitDone{});
         split_sites.assign(sites, SplitSite{});
-        for (size_t i = 0; i < tensors.size(); ++i) tensor_at[tensors[i].offset] = static_cast<int>(i);
         return kOk;
     }
 
-    int c_head() const { return c.tie_embeddings ? emb : lm_head; }
-
-    // The call with the int8 path's scratch of its stream; rested: also where its matmul rests now.
+    // The call with the int8 path's scratch; rested: also where its matmul rests now.
     GemmCall with_split(const GemmCall& g, hipStream_t s, bool rested = false) const {
         GemmCall c = g;
-        // The layers' weight gradients stay on FP64: eight windows' epilogues, two column-ordered operands to split and copy,
-        // and long-tailed gradients to recompute take 4.3 ms where FP64 takes 3.4 (8960 x 1536 over 8 x 1024).
-        if (g.a_kind == 1 && g.C != G(c_head())) return c;
+        if (side_on && s == side) return c;  // the scratch is the step's stream's
+        // Weight gradients other than the head's stay on FP64, on either stream: eight windows' epilogues, two column-ordered
+        // operands to split and copy, and long-tailed gradients to recompute took 4.3 ms where FP64 takes 3.4 (8960 x
+        // 1536 over 8 x 1024).
+        if (g.a_kind == 1 && g.C != G(head_id())) return c;
         if (split_stat != nullptr && g.split_site >= 0) {
             if (!rested && split_sites[static_cast<size_t>(g.split_site)].rest > 0) return c;
             c.split_stat = reinterpret_cast<uint32_t*>(split_stat + g.split_site);
         }
-        const int k = side_on && s == side ? 1 : 0;
-        c.split_scratch = split_mem[k];
-        c.split_cap = split_cap[k];
+        c.split_scratch = split_mem;
+        c.split_cap = split_cap;
         return c;
     }
 
@@ -1001,12 +998,12 @@ struct dllm_hip_trainer {
         return profile_end(flops_of(g), s);
     }
 
-    // Matmuls that share operand `share` (1: A, 2: B), back to back on one stream: it is split once.
-    int gemm_shared(const GemmCall* calls, int n, int share, hipStream_t s) {
+    // Matmuls that share their A operand, back to back on one stream: it is split once.
+    int gemm_shared(const GemmCall* calls, int n, hipStream_t s) {
         bool ready = false;
         for (int k = 0; k < n; ++k) {
             GemmCall g = calls[k];
-            g.split_share = share;
+            g.split_share = 1;
             g.split_ready = ready;
             const int64_t rows = gemm_split_rows(with_split(g, s));
             DLLM_TRY(gemm(g, s));
@@ -1177,7 +1174,7 @@ struct dllm_hip_trainer {
         const GemmCall calls[3] = {fwd_call(sv.h1, R, H, L.q, Popt(L.qb), sv.q_raw, nullptr),
                                    fwd_call(sv.h1, R, H, L.k, Popt(L.kb), sv.k_raw, nullptr),
                                    fwd_call(sv.h1, R, H, L.v, Popt(L.vb), sv.v, nullptr)};
-        return gemm_shared(calls, 3, 1, s);
+        return gemm_shared(calls, 3, s);
     }
 
     // out[R][N] (+)= x[R][K] @ W^T (+ bias); the matmul reads x itself (A transposed: A[k][r] = x[r][k]).
@@ -1268,8 +1265,7 @@ struct dllm_hip_trainer {
         g.nseg = nseg;
         g.l0 = 0;
         g.l1 = seg ? rows : seg_host.back();
-        const auto at = tensor_at.find(out - grads.as<float>());
-        if (at != tensor_at.end()) g.split_site = 3 * at->second + 2;
+        if (out == G(head_id())) g.split_site = 3 * head_id() + 2;
         if (!seg)
             for (size_t w = 0; w + 1 < seg_host.size(); ++w)
                 g.seg_max = std::max(g.seg_max, seg_host[w + 1] - seg_host[w]);
@@ -1474,7 +1470,7 @@ struct dllm_hip_trainer {
         } else {
             const GemmCall calls[2] = {fwd_call(sv.h2, R, H, L.gate, nullptr, sv.gate, nullptr),
                                        fwd_call(sv.h2, R, H, L.up, nullptr, sv.up, nullptr)};
-            DLLM_TRY(gemm_shared(calls, 2, 1, s));
+            DLLM_TRY(gemm_shared(calls, 2, s));
         }
         DLLM_TRY(launch_swiglu_forward(sv.gate, sv.up, sv.gate_act, sv.product, R * I, s, act()));
         if (post_norms()) {  // x_out = x_mid + post_norm(mlp)
@@ -1512,13 +1508,8 @@ struct dllm_hip_trainer {
             DLLM_TRY(side_wait(kSideMlp, s));  // the previous layer's gate and up dW read dgate, dup
             DLLM_TRY(launch_swiglu_backward(sv.gate, sv.up, sv.gate_act, dproduct, dgate, dup, R * I, s, act()));
             DLLM_TRY(side_fork_from(s, &ws));
-            {
-                GemmCall calls[2];
-                int n = 0;
-                if (grad_wanted(G(L.gate))) calls[n++] = dw_call(dgate, I, sv.h2, H, nseg, G(L.gate), nullptr, nullptr);
-                if (grad_wanted(G(L.up))) calls[n++] = dw_call(dup, I, sv.h2, H, nseg, G(L.up), nullptr, nullptr);
-                DLLM_TRY(gemm_shared(calls, n, 2, ws));
-            }
+            DLLM_TRY(linear_dw(dgate, I, sv.h2, H, nseg, G(L.gate), nullptr, nullptr, ws));
+            DLLM_TRY(linear_dw(dup, I, sv.h2, H, nseg, G(L.up), nullptr, nullptr, ws));
             DLLM_TRY(side_mark(kSideMlp));
             DLLM_TRY(side_wait(kSideNormMlp, s));  // the previous layer's mlp norm dW reads dh
             if (grouped(l, kGrpMlpDx, R)) {
@@ -1581,17 +1572,9 @@ struct dllm_hip_trainer {
         const int bs_[3] = {L.qb, L.kb, L.vb};
         const int64_t ns[3] = {QD, KVD, KVD};
         DLLM_TRY(side_fork_from(s, &ws));
-        {
-            GemmCall calls[3];
-            int n = 0;
-            for (int p = 0; p < 3; ++p) {
-                if (!grad_wanted(G(ws_[p]))) continue;
-                calls[n] = dw_call(ds[p], ns[p], sv.h1, H, nseg, G(ws_[p]), nullptr, nullptr);
-                calls[n++].seg_rowscale = unfold_scale(ws_[p]);
-            }
-            DLLM_TRY(gemm_shared(calls, n, 2, ws));
-        }
         for (int p = 0; p < 3; ++p) {
+            DLLM_TRY(linear_dw(ds[p], ns[p], sv.h1, H, nseg, G(ws_[p]), nullptr, nullptr, ws, nullptr, -1,
+                               unfold_scale(ws_[p])));
             if (bs_[p] >= 0 && grad_wanted(G(bs_[p])))
                 DLLM_TRY(launch_column_sums(0, ds[p], nullptr, nullptr, ns[p], seg_host.data(), nseg,
                                             ws == s ? col_part : col_part_side, G(bs_[p]), ws, window_weights(),
@@ -2056,7 +2039,7 @@ struct dllm_hip_trainer {
                                          router_loss_w, router_scale != 0.0 ? grad_row : nullptr, s));
         }
         DLLM_TRY(launch_rms_norm(x_final, P(final_norm), hidden, R, H, eps, uo(), nullptr, s));
-        const int head = c.tie_embeddings ? emb : lm_head;
+        const int head = head_id();
         DLLM_TRY(linear_fwd(hidden, R, H, head, nullptr, logits, nullptr, s));
         // loss and the head (backprop.py:174-206): Granite's logits scaling divides the logits and their gradient
         const bool logit_div = c.logits_scaling != 1.0;
