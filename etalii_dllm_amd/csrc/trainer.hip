@@ -946,7 +946,13 @@ struct dllm_hip_trainer {
         const size_t keep = size_t{2} << 30, left = free_bytes > keep ? free_bytes - keep : 0;
         split_cap = std::min({split_bytes(), kSplitMax, left});
         if (split_cap == 0) return kOk;
-        DLLM_TRY(make(&split_mem, split_cap));
+        if (make(&split_mem, split_cap) != kOk) {  // another process took the memory meanwhile
+            (void)hipGetLastError();
+            owned.pop_back();
+            split_mem = nullptr;
+            split_cap = 0;
+            return kOk;
+        }
         const size_t sites = 3 * tensors.size();
         DLLM_TRY(make(&split_stat, sites));
         DLLM_TRY(check_hip(hipMemset(split_stat, 0, sites * sizeof(SplitDone)), "memset"));
