@@ -54,8 +54,13 @@ def assert_same(a: np.ndarray, b: np.ndarray, what: str) -> None:
 
 
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("rows,inf,outf", [(2049, 1540, 4868), (1000, 8196, 1348), (4100, 516, 5444)])
-def test_linear(K, kind, rows, inf, outf):
+@pytest.mark.parametrize("rows,inf,outf,int8", [(2049, 1540, 4868, True), (1300, 8196, 1348, True), (4100, 644, 5444, True),
+                                                (1000, 8196, 1348, False), (4100, 516, 5444, False)])
+def test_linear(K, kind, rows, inf, outf, int8):
+    """int8: which path the whole call takes (the pieces are all FP64's)."""
+    h = M.load()
+    assert bool(h.matmul_rows(C.byref(M.row_major(rows, outf, inf)))) == int8
+    assert not h.matmul_rows(C.byref(M.row_major(256, 512, inf)))
     x, w = operand(kind, 1, rows, inf), operand("gauss" if kind == "special" else kind, 2, outf, inf)
     b = operand("gauss", 3, 1, outf)[0]
     got = K.linear(x, w, b)
@@ -71,6 +76,10 @@ def test_linear(K, kind, rows, inf, outf):
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("rows,inf,outf", [(2051, 900, 4868), (8191, 1028, 1540)])
 def test_linear_backward(K, kind, rows, inf, outf):
+    h = M.load()
+    assert h.matmul_rows(C.byref(M.row_major(rows, inf, outf, b_t=False))) and h.matmul_rows(C.byref(M.windowed(outf, inf, rows)))
+    assert not h.matmul_rows(C.byref(M.row_major(128, inf, outf, b_t=False)))
+    assert not h.matmul_rows(C.byref(M.windowed(128, inf, rows)))
     x, w = operand("gauss", 4, rows, inf), operand("gauss", 5, outf, inf)
     dy = operand(kind, 6, rows, outf)
     dx, dw, db = K.linear_backward(x, w, dy, with_bias=True)
