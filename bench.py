@@ -29,22 +29,23 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 FP64_PEAK_TFLOPS = 78.6  # MI355X dense FP64 (vector FMA and matrix alike)
+INT8_EXACT_TFLOPS = 181.0  # 19 int8 digit products per multiply-add, at the 3440 TOP/s that random digits sustain
 
 CONFIGS = {
-    # the metric's workload
+    # the workload of the metric
     "c3": dict(name="Qwen2.5-1.5B", vocab=151936, hidden=1536, intermediate=8960, layers=28, heads=12, kv_heads=2,
                head_dim=128, rms_norm_eps=1e-6, rope_theta=1e6, tie_embeddings=True, attention_bias=True,
                batch=8, seq=1024),
-    # the reference's CPU-runnable case
+    # the case that the reference runs on a CPU
     "c1": dict(name="SmolLM2-135M", vocab=49152, hidden=576, intermediate=1536, layers=30, heads=9, kv_heads=3,
                head_dim=64, rms_norm_eps=1e-5, rope_theta=1e5, tie_embeddings=True, attention_bias=False,
                batch=4, seq=256),
-    # BASELINE.json configs[3]: LoRA (rank 16, alpha 32, q k v o gate up down; A ~ N(0, 0.02), B = 0) on a Q8_0 base
+    # LoRA (rank 16, alpha 32, q k v o gate up down; A ~ N(0, 0.02), B = 0) on a Q8_0 base
     "c4": dict(name="Qwen3-0.6B LoRA on a Q8_0 base", vocab=151936, hidden=1024, intermediate=3072, layers=28,
                heads=16, kv_heads=8, head_dim=128, rms_norm_eps=1e-6, rope_theta=1e6, tie_embeddings=True,
                attention_bias=False, qk_norm=1, batch=8, seq=2048,
                lora=dict(rank=16, alpha=32.0, targets=("q", "k", "v", "o", "gate", "up", "down"))),
-    # BASELINE.json configs[4]: routed experts with the load-balancing loss (router_aux_loss 0.01)
+    # routed experts with the load-balancing loss (router_aux_loss 0.01)
     "c5": dict(name="OLMoE-1B-7B", vocab=50304, hidden=2048, intermediate=1024, layers=16, heads=16, kv_heads=16,
                head_dim=128, rms_norm_eps=1e-5, rope_theta=1e4, tie_embeddings=False, attention_bias=False,
                qk_norm=2, experts=64, experts_per_token=8, normalize_expert_weights=False, expert_intermediate=1024,
@@ -277,23 +278,28 @@ def _counter_rows(path: str, kernel_substring: str, counter: str) -> list[float]
     return out
 
 
+# a matmul is one launch of the first; on the int8 path the others run with it
+MATMUL_KERNELS = ("gemm_mfma_kernel", "split_clear_kernel", "split_top_kernel", "split_amax_kernel", "split_digits_kernel",
+                  "split_gemm_kernel", "split_fix_kernel", "split_sum_kernel")
+
+
 def traffic_summary(config: str, fetch_csv: str, write_csv: str, copy_fetch_csv: str, copy_write_csv: str) -> int:
-    """HBM bytes per matmul launch = mean(FETCH_SIZE) x fetch scale + mean(WRITE_SIZE) x write scale, the scales
-    being the copy kernel's known bytes over what the same counters read for it (counters are in KiB)."""
-    fetch = _counter_rows(fetch_csv, "gemm_mfma_kernel", "FETCH_SIZE")
-    write = _counter_rows(write_csv, "gemm_mfma_kernel", "WRITE_SIZE")
+    """HBM bytes per matmul = FETCH_SIZE x fetch scale + WRITE_SIZE x write scale of all its kernels, the scales being the
+    copy kernel's known bytes over what the same counters read for it (counters are in KiB)."""
+    launches = len(_counter_rows(fetch_csv, MATMUL_KERNELS[0], "FETCH_SIZE"))
+    fetch = sum(sum(_counter_rows(fetch_csv, k, "FETCH_SIZE")) for k in MATMUL_KERNELS) / launches
+    write = sum(sum(_counter_rows(write_csv, k, "WRITE_SIZE")) for k in MATMUL_KERNELS) / launches
     copy_fetch = max(_counter_rows(copy_fetch_csv, "copy", "FETCH_SIZE") or
                      _counter_rows(copy_fetch_csv, "elementwise", "FETCH_SIZE"))
     copy_write = max(_counter_rows(copy_write_csv, "copy", "WRITE_SIZE") or
                      _counter_rows(copy_write_csv, "elementwise", "WRITE_SIZE"))
     fetch_scale = COPY_BYTES / (copy_fetch * 1024.0)
     write_scale = COPY_BYTES / (copy_write * 1024.0)
-    per_launch = (sum(fetch) / len(fetch) * 1024.0 * fetch_scale + sum(write) / len(write) * 1024.0 * write_scale)
+    per_launch = fetch * 1024.0 * fetch_scale + write * 1024.0 * write_scale
     path = ROOT / "profiles" / "gemm_traffic.json"
     data = json.loads(path.read_text()) if path.exists() else {}
-    data[config] = {"bytes_per_launch": per_launch, "launches": len(fetch), "fetch_scale": fetch_scale,
-                    "write_scale": write_scale, "fetch_kib_mean": sum(fetch) / len(fetch),
-                    "write_kib_mean": sum(write) / len(write)}
+    data[config] = {"bytes_per_launch": per_launch, "launches": launches, "fetch_scale": fetch_scale,
+                    "write_scale": write_scale, "fetch_kib_mean": fetch, "write_kib_mean": write}
     path.write_text(json.dumps(data, indent=1) + "\n")
     print(json.dumps(data[config]))
     return 0
@@ -539,8 +545,8 @@ def main() -> int:
     from etalii_dllm_amd.trainer import Decoder, Trainer
 
     lib.dllm_hip_trainer_profile.argtypes = [C.c_void_p, C.c_int]
-    lib.dllm_hip_trainer_profile_read.argtypes = [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_double),
-                                                  C.POINTER(C.c_double)]
+    for read in (lib.dllm_hip_trainer_profile_read, lib.dllm_hip_trainer_profile_read_int8):
+        read.argtypes = [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_double), C.POINTER(C.c_double)]
     decoder = Decoder(cfg["vocab"], cfg["hidden"], cfg["intermediate"], cfg["layers"], cfg["heads"], cfg["kv_heads"],
                       cfg["head_dim"], cfg["rms_norm_eps"], cfg["rope_theta"], cfg["tie_embeddings"],
                       cfg["attention_bias"], cfg.get("qk_norm", 0), 0, cfg.get("experts", 0),
@@ -586,6 +592,8 @@ def main() -> int:
     roof_elapsed = time.perf_counter() - t_roof
     launches, ms, flops = C.c_int64(), C.c_double(), C.c_double()
     check(lib.dllm_hip_trainer_profile_read(trainer.handle, C.byref(launches), C.byref(ms), C.byref(flops)))
+    int8 = (C.c_int64(), C.c_double(), C.c_double())
+    check(lib.dllm_hip_trainer_profile_read_int8(trainer.handle, *map(C.byref, int8)))
     check(lib.dllm_hip_trainer_profile(trainer.handle, 0))
     if args.export_timing:
         for kind, what in ((0, "model.dllm data"), (1, "checkpoint data")):
@@ -596,6 +604,15 @@ def main() -> int:
     trainer.close()
     ms_per_step = elapsed * 1000.0 / args.steps
     achieved = flops.value / (ms.value * 1e9) if ms.value > 0 else None  # TFLOP/s
+    # each path's flop at its own peak
+    peak = FP64_PEAK_TFLOPS
+    paths = {}
+    if flops.value > 0:
+        parts = {"fp64": (launches.value - int8[0].value, ms.value - int8[1].value, flops.value - int8[2].value),
+                 "int8": tuple(v.value for v in int8)}
+        paths = {k: {"launches": n, "ms": t, "achieved": f / (t * 1e9) if t > 0 else None,
+                     "peak": FP64_PEAK_TFLOPS if k == "fp64" else INT8_EXACT_TFLOPS} for k, (n, t, f) in parts.items()}
+        peak = flops.value / sum(f / paths[k]["peak"] for k, (_, _, f) in parts.items())
     if roofline_steps:
         log(f"matmuls: {launches.value} launches over {roofline_steps} steps, {ms.value:.1f} ms, {flops.value:.3e} "
             f"flop ({100.0 * ms.value / (roof_elapsed * 1000.0):.1f}% of those steps' time, "
@@ -627,12 +644,13 @@ def main() -> int:
                                                      "full fine-tune step (forward, backward, global-norm clip, AdamW)"),
                    "global_batch": cfg["batch"], "seq_len": cfg["seq"], "parallelism": "single GPU",
                    "layers": cfg["layers"], "hidden": cfg["hidden"], "vocab": cfg["vocab"]},
-        "roofline": {"bound": "mfma", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / FP64_PEAK_TFLOPS if achieved else None, "traffic": traffic,
-                     "note": "peak is FP64's; large matmuls run on the int8 matrix cores (19 exact digit products each)",
-                     "kernel": "gemm_mfma_kernel (FP64 MFMA matmul, every launch of the matmul-timing steps)",
-                     "timing_steps": roofline_steps,
-                     "step_fraction_of_peak": matmul_flops_per_step(cfg) / (ms_per_step * 1e9) / FP64_PEAK_TFLOPS},
+        "roofline": {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
+                     "frac": achieved / peak if achieved else None, "traffic": traffic,
+                     "note": "peak: each path's flop at its own rate, FP64's and that of 19 int8 digit products each",
+                     "kernel": "the step's matmuls: gemm_mfma_kernel (FP64) and, for large ones, split_gemm_kernel (int8, with "
+                               "its splitting and recomputation); every one of the matmul-timing steps",
+                     "paths": paths, "timing_steps": roofline_steps,
+                     "step_fraction_of_peak": matmul_flops_per_step(cfg) / (ms_per_step * 1e9) / peak},
         "cpu_baseline": baseline,
     }
     print(json.dumps(result), flush=True)

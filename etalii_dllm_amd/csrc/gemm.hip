@@ -711,7 +711,7 @@ __device__ __forceinline__ void maccumulate(const GemmParams& p, MStage<kA, kBI,
         // Every wave's reads of the stage have returned before the next issue overwrites it. The wait is needed: the
         // compiler places the stage's last MFMAs, and the waits for their fragments, after this barrier, and reads only
         // issued could be overtaken by a copy that another wave issues after it (a step of 450 such launches gave other
-        // weights about once in a hundred; the wait costs 0.5% of these launches).
+        // weights about once in fifty; the wait costs 0.5% of the large launches).
         workgroup_barrier();
     }
     if (tail) {

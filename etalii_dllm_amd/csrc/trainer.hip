@@ -891,17 +891,21 @@ struct dllm_hip_trainer {
     // ---- matmul timing (dllm_hip_trainer_profile) ----
     bool profiling = false;
     std::vector<hipEvent_t> events;  // pairs
+    std::vector<char> event_path;    // each pair's path: 0 FP64, 1 int8
     size_t event_used = 0;
-    double profile_flops = 0.0;
-    int64_t profile_launches = 0;
-    double profile_ms_done = 0.0;
+    struct PathTotals {
+        double flops = 0.0;
+        int64_t launches = 0;
+        double ms_done = 0.0;
+    };
+    PathTotals profile_totals[2];  // by path
 
     int drain_events() {
         for (size_t i = 0; i + 1 < event_used; i += 2) {
             DLLM_TRY(check_hip(hipEventSynchronize(events[i + 1]), "event"));
             float ms = 0.0f;
             DLLM_TRY(check_hip(hipEventElapsedTime(&ms, events[i], events[i + 1]), "event"));
-            profile_ms_done += ms;
+            profile_totals[static_cast<int>(event_path[i / 2])].ms_done += ms;
         }
         event_used = 0;
         return kOk;
@@ -991,7 +995,8 @@ struct dllm_hip_trainer {
     }
 
     int gemm(const GemmCall& g, hipStream_t s) {
-        if (split_stat != nullptr && g.split_site >= 0 && gemm_split_rows(with_split(g, s)) > 0) {
+        const bool int8 = gemm_split_rows(with_split(g, s)) > 0;
+        if (int8 && split_stat != nullptr && g.split_site >= 0) {
             SplitSite& site = split_sites[static_cast<size_t>(g.split_site)];
             SplitCost cost = gemm_split_cost(with_split(g, s));
             cost.fp64 += site.cost.fp64;
@@ -1001,7 +1006,7 @@ struct dllm_hip_trainer {
         if (!profiling) return launch_gemm(with_split(g, s), s);
         DLLM_TRY(profile_begin(s));
         DLLM_TRY(launch_gemm(with_split(g, s), s));
-        return profile_end(flops_of(g), s);
+        return profile_end(flops_of(g), int8 ? 1 : 0, s);
     }
 
     // Matmuls that share their A operand, back to back on one stream: it is split once.
@@ -1023,7 +1028,7 @@ struct dllm_hip_trainer {
         if (!profiling) return launch_gemm_group(grp, table, s);
         DLLM_TRY(profile_begin(s));
         DLLM_TRY(launch_gemm_group(grp, table, s));
-        return profile_end(flops, s);
+        return profile_end(flops, 0, s);
     }
 
     static double flops_of(const GemmCall& g) {
@@ -1038,16 +1043,18 @@ struct dllm_hip_trainer {
                 hipEvent_t e;
                 DLLM_TRY(check_hip(hipEventCreate(&e), "event"));
                 events.push_back(e);
+                event_path.resize((events.size() + 1) / 2);
             }
         }
         return check_hip(hipEventRecord(events[event_used], s), "event");
     }
 
-    int profile_end(double flops, hipStream_t s) {
+    int profile_end(double flops, int path, hipStream_t s) {
         DLLM_TRY(check_hip(hipEventRecord(events[event_used + 1], s), "event"));
+        event_path[event_used / 2] = static_cast<char>(path);
         event_used += 2;
-        profile_flops += flops;
-        profile_launches += 1;
+        profile_totals[path].flops += flops;
+        profile_totals[path].launches += 1;
         return kOk;
     }
 
@@ -2555,9 +2562,7 @@ int dllm_hip_trainer_profile(dllm_hip_trainer* t, int enable) {
     DLLM_TRY(t->drain_events());
     t->profiling = enable != 0;
     if (t->profiling) {
-        t->profile_flops = 0.0;
-        t->profile_launches = 0;
-        t->profile_ms_done = 0.0;
+        for (auto& p : t->profile_totals) p = {};
     }
     return kOk;
 }
@@ -2565,9 +2570,20 @@ int dllm_hip_trainer_profile(dllm_hip_trainer* t, int enable) {
 int dllm_hip_trainer_profile_read(dllm_hip_trainer* t, int64_t* launches, double* ms, double* flops) {
     DLLM_REQUIRE(t, "null argument");
     DLLM_TRY(t->drain_events());
-    if (launches) *launches = t->profile_launches;
-    if (ms) *ms = t->profile_ms_done;
-    if (flops) *flops = t->profile_flops;
+    const auto& p = t->profile_totals;
+    if (launches) *launches = p[0].launches + p[1].launches;
+    if (ms) *ms = p[0].ms_done + p[1].ms_done;
+    if (flops) *flops = p[0].flops + p[1].flops;
+    return kOk;
+}
+
+int dllm_hip_trainer_profile_read_int8(dllm_hip_trainer* t, int64_t* launches, double* ms, double* flops) {
+    DLLM_REQUIRE(t, "null argument");
+    DLLM_TRY(t->drain_events());
+    const auto& p = t->profile_totals[1];
+    if (launches) *launches = p.launches;
+    if (ms) *ms = p.ms_done;
+    if (flops) *flops = p.flops;
     return kOk;
 }
 

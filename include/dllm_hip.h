@@ -400,9 +400,12 @@ int dllm_hip_trainer_log_probabilities(dllm_hip_trainer* trainer, const int64_t*
 
 /* Matmul timing inside steps: with profiling on, every matmul launch of the trainer is bracketed by HIP events on its
  * stream; _read sums them (waiting for the events) into the number of launches, their total milliseconds and their
- * algorithmic flops (2 * rows * columns * reduction length each). Enabling resets the totals. */
+ * algorithmic flops (2 * rows * columns * reduction length each); _read_int8 gives the part of them that ran on the int8
+ * matrix cores, with the splitting and recomputation there. Enabling resets the totals. */
 int dllm_hip_trainer_profile(dllm_hip_trainer* trainer, int enable);
 int dllm_hip_trainer_profile_read(dllm_hip_trainer* trainer, int64_t* launches, double* milliseconds, double* flops);
+int dllm_hip_trainer_profile_read_int8(dllm_hip_trainer* trainer, int64_t* launches, double* milliseconds,
+                                       double* flops);
 
 /* ---- model and checkpoint files (src/etalii_dllm/modelfile.py, training/trainer.py:477-630) ----
  * kind 0: model.dllm (write_model_file, modelfile.py:68-136): prefix "DLLM", u32 1, u64 header length; the data

@@ -115,7 +115,7 @@ def test_a_resting_matmul_runs_grouped_and_comes_back(other_rows, hot_rows):
 
     lib = kernels.lib
     h = M.load()
-    for n in (2048, 2044):  # of the layer's matmuls these two alone are the int8 path's
+    for n in (2048, 2044):  # of the layer's matmuls gate, up and down's input gradient are the int8 path's
         assert h.matmul_rows(C.byref(M.row_major(n, 3712, 896))) == n
         assert not any(h.matmul_rows(C.byref(M.row_major(n, *s))) for s in ((896, 3712), (896, 896)))
     t = Trainer(Decoder(256, 896, 3712, 1, 14, 2, 64, 1e-6, 1e4, True), 2048, 2, 1024)
@@ -134,24 +134,31 @@ def test_a_resting_matmul_runs_grouped_and_comes_back(other_rows, hot_rows):
     windows = {n: [tokens[:1025], tokens[1024:n + 1]] for n in (2048, 2044)}
     step = 0
 
-    def launches(rows: int) -> int:
+    def launches(rows: int) -> tuple[int, int]:
+        """A step's matmul launches, and those of them on the int8 path."""
         nonlocal step
         step += 1
         kernels.check(lib.dllm_hip_trainer_profile(t.handle, 1))
         t.step(windows[rows], 0.0, step, weight_decay=0.0)
-        n, ms, flops = C.c_int64(), C.c_double(), C.c_double()
-        kernels.check(lib.dllm_hip_trainer_profile_read(t.handle, C.byref(n), C.byref(ms), C.byref(flops)))
-        return n.value
+        seen = []
+        for read in reads:
+            n, ms, flops = C.c_int64(), C.c_double(), C.c_double()
+            kernels.check(read(t.handle, C.byref(n), C.byref(ms), C.byref(flops)))
+            assert (ms.value > 0.0 and flops.value > 0.0) == (n.value > 0)
+            seen.append(n.value)
+        return tuple(seen)
 
     lib.dllm_hip_trainer_profile.argtypes = [C.c_void_p, C.c_int]
-    lib.dllm_hip_trainer_profile_read.argtypes = [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_double),
-                                                  C.POINTER(C.c_double)]
+    reads = [lib.dllm_hip_trainer_profile_read, lib.dllm_hip_trainer_profile_read_int8]
+    for read in reads:
+        read.argtypes = [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_double), C.POINTER(C.c_double)]
     t.load(weights)
     apart = launches(2048)
+    assert apart[1] == 3
     t.load(hot)
     assert launches(2048) == apart  # hands its tiles back
     t.load(weights)
     rows = 2044 if other_rows else 2048
-    assert [launches(rows) for _ in range(32)] == [apart - 1] * 32  # gate and up in one launch
+    assert [launches(rows) for _ in range(32)] == [(apart[0] - 1, 1)] * 32  # gate and up in one launch
     assert [launches(rows) for _ in range(3)] == [apart] * 3
     t.close()
