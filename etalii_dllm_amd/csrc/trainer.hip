@@ -994,18 +994,19 @@ struct dllm_hip_trainer {
         return check_hip(hipMemsetAsync(split_stat, 0, split_done.size() * sizeof(SplitDone), s), "memset");
     }
 
-    int gemm(const GemmCall& g, hipStream_t s) {
-        const bool int8 = gemm_split_rows(with_split(g, s)) > 0;
-        if (int8 && split_stat != nullptr && g.split_site >= 0) {
+    int gemm(const GemmCall& call, hipStream_t s) {
+        const GemmCall g = with_split(call, s);
+        const bool int8 = g.split_scratch != nullptr && gemm_split_rows(g) > 0;
+        if (int8 && g.split_site >= 0) {
             SplitSite& site = split_sites[static_cast<size_t>(g.split_site)];
-            SplitCost cost = gemm_split_cost(with_split(g, s));
+            SplitCost cost = gemm_split_cost(g);
             cost.fp64 += site.cost.fp64;
             cost.split += site.cost.split;
             site.cost = cost;
         }
-        if (!profiling) return launch_gemm(with_split(g, s), s);
+        if (!profiling) return launch_gemm(g, s);
         DLLM_TRY(profile_begin(s));
-        DLLM_TRY(launch_gemm(with_split(g, s), s));
+        DLLM_TRY(launch_gemm(g, s));
         return profile_end(flops_of(g), int8 ? 1 : 0, s);
     }
 
