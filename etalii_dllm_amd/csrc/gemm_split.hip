@@ -21,9 +21,9 @@
 //   Otherwise the output goes to a list, and split_fix_kernel computes its chain: one output in 2500 on Gaussian operands
 //   at L = 1536, one in 260 at 8192 with rows and columns of unequal size. A tile of which more than one in 64 would go
 //   there (rows of very wide dynamic range, infinities, NaNs) is flagged and recomputed whole by the FP64 matmul.
-//   Measured: 1023 x 8960 x 1536 in 265 us of 380 for the call, against 600 in FP64; 8192 x 1536 x 8960 in 1.67 ms (135
-//   TFLOP/s), with splitting and recomputation 2.5, against 3.3. The matrix cores' power bounds it: random digits hold the
-//   clock at 1.7 GHz with them busy throughout, 181 TFLOP/s.
+//   Measured: 1023 x 8960 x 1536 in 269 us of 371 for the call, against 600 in FP64 (matrix cores 43% busy at 2.26 GHz: 4.4
+//   rounds of workgroups and their epilogues); 8192 x 1536 x 8960 in 1.69 ms (133 TFLOP/s, 70% busy at 1.72 GHz: power
+//   lowers the clock, and random digits on registers alone reach 181), with splitting and recomputation 2.5, against 3.5.
 #include <algorithm>
 
 #include "common.h"
