@@ -394,7 +394,7 @@ C2_SWEEP = (1, 7, 64, 2048, 8192)
 
 
 def c2_microbench(iters: int = 20) -> int:
-    """the per-op backward kernels at Qwen2.5-0.5B layer shapes through the C ABI on
+    """The per-op backward kernels at Qwen2.5-0.5B layer shapes through the C ABI on
     device-resident inputs (weights N(0, 0.02), activations N(0, 1), upstream gradients N(0, 1e-3)), at each row count
     M of the sweep: the layer's seven linear_backward calls (dX and dW), dX and dW of the gate projection alone,
     rms_norm_backward, the RoPE backward of q and k, silu_backward over the SwiGLU width, causal GQA
