@@ -942,12 +942,12 @@ struct dllm_hip_trainer {
         return most;
     }
 
-    // The int8 path's scratch, after everything else and of the memory that is left, 2 GiB kept free: a trainer that fits
-    // without it is made without it, and its matmuls then run in smaller row blocks or in FP64.
+    // The int8 path's scratch, after everything else and of the memory that is left above 2 GiB at most half (the rest is the
+    // caller's): a trainer that fits without it is made without it, and its matmuls then run in smaller row blocks or in FP64.
     int split_setup() {
         size_t free_bytes = 0, total_bytes = 0;
         DLLM_TRY(check_hip(hipMemGetInfo(&free_bytes, &total_bytes), "hipMemGetInfo"));
-        const size_t keep = size_t{2} << 30, left = free_bytes > keep ? free_bytes - keep : 0;
+        const size_t keep = size_t{2} << 30, left = free_bytes > keep ? (free_bytes - keep) / 2 : 0;
         split_cap = std::min({split_bytes(), kSplitMax, left});
         if (split_cap == 0) return kOk;
         if (make(&split_mem, split_cap) != kOk) {  // another process took the memory meanwhile

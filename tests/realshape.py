@@ -8,7 +8,7 @@ digests of every gradient, parameter and AdamW moment after each step (tests/gol
 test regenerates the same inputs, runs the same steps on the GPU and compares digests. Equal SHA-256 digests are equal
 bits.
 
-Shapes follow BASELINE's configurations (SmolLM2-135M, Qwen2.5-1.5B, Qwen3-0.6B with LoRA on a Q8_0 base, OLMoE-1B-7B),
+Shapes follow the benchmark's configurations (SmolLM2-135M, Qwen2.5-1.5B, Qwen3-0.6B with LoRA on a Q8_0 base, OLMoE-1B-7B),
 plus Gemma-2-2B's layer (256-wide heads, soft-caps, sandwich norms, vocabulary 256000) Qwen1.5-MoE-A2.7B's (60
 experts and a gated shared expert) and OLMo-2-1B's (post norms), with fewer layers where the full depth only repeats the same launches; the vocabulary, hidden size, heads,
 intermediate sizes, window lengths and expert counts are the real ones, so every size-selected code path of the step
