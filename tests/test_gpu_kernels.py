@@ -185,7 +185,7 @@ def test_elementwise(K, ora):
 @pytest.mark.parametrize(("rows", "vocab"), [(6, 301), (3, 5000), (2, 49152), (6, 1024), (5, 515), (9, 2049),
                                              (6, 151936)])
 def test_cross_entropy(K, ora, rows, vocab):
-    """Row counts that do and do not fill the 4-row waves; vocabularies of whole 512-column chunks, a partial last
+    """Row counts that do and do not fill the workgroups' two rows; vocabularies of whole 512-column chunks, a partial last
     chunk, one that is not a multiple of 4 (the scalar loads) and the full 151936."""
     logits = O.gaussian(16, rows, vocab, scale=4.0)
     targets = np.array([3, -1, vocab - 1, 0, 17, 17, 5, -1, 2][:rows], np.int64)
@@ -193,6 +193,24 @@ def test_cross_entropy(K, ora, rows, vocab):
     lb, db = ora.cross_entropy(logits, targets, 0.25)
     assert la == lb
     assert_same(da, db, "dlogits")
+
+
+@pytest.mark.parametrize("rows", [1, 2, 7, 2047, 2048, 2051])
+@pytest.mark.parametrize("vocab", [1, 3, 511, 1028])
+def test_cross_entropy_either_side_of_the_row_limit(K, ora, rows, vocab):
+    """Below 2048 rows two per workgroup with a wave that only adds, from there on four per wave; rows with infinities and
+    NaNs among ordinary ones."""
+    for special in (False, True):
+        logits = O.gaussian(18, rows, vocab, scale=4.0).reshape(rows, vocab)
+        if special:
+            for r, (at, value) in enumerate([(0, np.nan), (-1, np.nan), (vocab // 2, np.inf), (0, -np.inf)]):
+                logits[r::5, at] = value
+            logits[4::5] = -np.inf
+        targets = (np.arange(rows) % (vocab + 1) - 1).astype(np.int64)
+        la, da = K.cross_entropy(logits, targets, 0.25)
+        lb, db = ora.cross_entropy(logits, targets, 0.25)
+        assert la == lb or (np.isnan(la) and np.isnan(lb))
+        assert_same_or_nan(da, db, "dlogits")
 
 
 def test_cross_entropy_rejects_target_out_of_range(K):
